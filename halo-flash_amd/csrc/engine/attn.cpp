@@ -1,6 +1,7 @@
 // Decode attention dispatch (FlashNextGpu::Attention, src/engine/flash_next_gpu.cpp:581-680, and the batched
 // per-entry attention of StepBatch): paged KV, prefix read once per step for all sessions.
 #include <algorithm>
+#include <array>
 #include <vector>
 
 #include "engine.hpp"
@@ -137,23 +138,29 @@ int halo_op_attn_prefill(halo_engine* eng, const halo_paged_kv* kv, const halo_p
   if (segs == nullptr || nseg == 0 || q == nullptr || gate == nullptr || (o == nullptr && oq == nullptr) ||
       ((oq == nullptr) != (os == nullptr)))
     return SetErr(err, errlen, "attn prefill: missing arguments"), -1;
-  std::vector<std::uint32_t> tiles;
+  // 16-token tiles, or 8-token ones (the output dims split over two waves) where those still fit the 256 CUs once
+  std::uint64_t tiles8 = 0;
+  for (std::uint32_t i = 0; i < nseg; ++i) tiles8 += CeilDiv(segs[i].length, 8);
+  const std::uint32_t tile = tiles8 * kv->kv_heads <= 256 ? 8 : 16;
+  std::vector<std::array<std::uint32_t, 4>> tiles;
   for (std::uint32_t i = 0; i < nseg; ++i) {
     const halo_prefill_segment& g = segs[i];
     if (g.session >= kv->sessions || g.length == 0 || g.start + g.length > kv->max_context)
       return SetErr(err, errlen, "attn prefill: segment %u (session %u, %u + %u) out of range", i, g.session, g.start,
                     g.length),
              -1;
-    for (std::uint32_t k = 0; k < g.length; k += 8)
-      tiles.insert(tiles.end(), {g.first + k, std::min<std::uint32_t>(8, g.length - k), g.session, g.start + k});
+    for (std::uint32_t k = 0; k < g.length; k += tile)
+      tiles.push_back({g.first + k, std::min<std::uint32_t>(tile, g.length - k), g.session, g.start + k});
   }
-  const std::size_t need = tiles.size() * sizeof(std::uint32_t);
+  // longest first: a block's work grows with its tile's position, and blocks start in grid order
+  std::stable_sort(tiles.begin(), tiles.end(), [](const auto& a, const auto& b) { return a[3] + a[1] > b[3] + b[1]; });
+  const std::size_t need = tiles.size() * sizeof(tiles[0]);
   if (ws == nullptr || ws_bytes < need) return SetErr(err, errlen, "attn prefill: workspace %zu < %zu", ws_bytes, need), -1;
   halo_buffer b{ws, need, nullptr};
   if (halo_upload(halo_engine_device(eng), &b, 0, tiles.data(), need, err, errlen) != 0) return -1;
   const halo_arg a[] = {Ptr(q), Ptr(gate), Ptr(kv->k_pool), Ptr(kv->v_pool), Ptr(kv->pages), Ptr(ws), Ptr(o), Ptr(oq),
                         Ptr(os), U32(Hq), U32(kv->kv_heads), U32(kv->max_pages)};
-  return Launch(eng, "halo_attn_prefill", D3(static_cast<std::uint32_t>(tiles.size() / 4), kv->kv_heads), D3(256), a,
+  return Launch(eng, tile == 8 ? "halo_attn_prefill_d2" : "halo_attn_prefill", D3(static_cast<std::uint32_t>(tiles.size() * kv->kv_heads)), D3(256), a,
                 err, errlen);
 }
 

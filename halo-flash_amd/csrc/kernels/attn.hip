@@ -677,253 +677,423 @@ extern "C" __global__ void __launch_bounds__(64)
 // ---- causal GQA attention for a ragged batch of prefill tokens (split-fp16 MFMA) -----------------------------------
 // Reference semantics: ReferenceModel::Attention (src/model/reference.cpp:368-416, 492-527) for every token of a
 // prompt: softmax(q . K[0..p]^T / sqrt(d)) V[0..p] * sigmoid(gate), K / V already appended at the tokens' positions.
-// tiles [n][4] = {first token index in the batch, tokens (<= 8), session, position of the first token}; a tile's
-// tokens are consecutive positions of one session. Block (tile, kv head): 64 queries = 8 tokens x G = 8 q heads,
-// wave w the tokens 2w, 2w + 1 (query row r = 8 (token - 2w) + g). Per 32-key chunk: scores on
-// the matrix cores (A = q rows kept in registers, B = K chunk in LDS), online softmax per row in the MFMA output
-// layout (a row's 32 scores sit in one 16-lane DPP row, two tiles), P through LDS, P V with the same MFMA (B = V
-// chunk in LDS). Output o (fp32, may be null) and its Q8 quantization oq / os (may be null), per token
-// [Hq * 256], after o /= l and o *= sigmoid(gate). q, gate [T][Hq][256].
+// tiles [n][4] = {first token index in the batch, tokens (<= 16), session, position of the first token}; a tile's
+// tokens are consecutive positions of one session. Output o (fp32, may be null) and its Q8 quantization oq / os (may
+// be null), per token [Hq * 256], after o /= l and o *= sigmoid(gate). q, gate [T][Hq][256]. G = Hq / Hkv = 8.
 //
 // Every fp32 operand x enters as a pair of halves, hi = fp16(x) and lo = fp16(x - hi) (|x - hi - lo| <= 2^-22 |x|
-// for normal values), and each product is formed as hi * hi + hi * lo + lo * hi on v_mfma_f32_16x16x32_f16
+// for normal values), and each product is formed as hi * hi + hi * lo + lo * hi on v_mfma_f32_32x32x16_f16
 // (products of halves are exact in the fp32 accumulator; the dropped lo * lo term is below 2^-22 of the product).
-// Three fp16 MFMAs cost 3/16 of the fp32 MFMA issue time of the same products, so the scores and P V run at about
-// five times the fp32 MFMA rate with fp32-level accuracy. q, k and V are scaled by 2^8 and the probabilities by 2^14
-// before the split (kSqk, kSvv, kSpp); a query row, K chunk or V chunk whose magnitude would overflow fp16 at 2^8
-// takes a smaller power of two (halo::SplitScale), so any finite operand range is accepted.
-// (An fp32 version of this kernel on v_mfma_f32_16x16x4f32 ran the C4 prefix prefill's attention at 78.8 TFLOP/s.)
-// The K and V chunks are converted once per block while staged in LDS: K as kh / kl [key][256] (16-byte chunk c of row key at
-// c ^ (key & 15): the 16 lanes reading one column of keys hit 16 different bank groups), V transposed as vh / vl
-// [dim][32 keys] (chunk c at c ^ ((dim >> 2) & 3)), so each MFMA operand is one 16-byte LDS read. The next chunk's
-// K and V are loaded into registers while the current chunk computes.
+// q, K and V are scaled by 2^8 and the probabilities by 2^10 before the split (kSqk, kSvv, kSppT); a query row, K chunk
+// or V chunk whose magnitude would overflow fp16 at 2^8 takes a smaller power of two (halo::SplitScale), so any finite
+// operand range is accepted.
+//
+// Block (tile, kv head): 128 queries = 16 tokens x 8 q heads; wave w the tokens 4 w .. 4 w + 3, query n = 8 (token -
+// 4 w) + head. Both products run transposed, so that a query is a column and stays in one lane pair (n, n + 32)
+// throughout: S^T = K Q^T (A = K chunk from LDS, B = the wave's queries, kept in registers) leaves each lane 16 of its
+// query's 32 scores, the softmax needs one exchange between the pair, and the probabilities are, in place, the B
+// operand of O^T += V^T P^T: its k order (lane half h, slot j -> key 16 s + 8 (j / 4) + 4 h + j % 4) is matched by the
+// order in which V's keys are read (ds_read_b64_tr_b16: 4 keys of one dim per lane from a row-major V chunk).
+//
+// 32-key chunks, double-buffered in LDS as halves (K and V, hi and lo, [key][256]: 128 KB); one barrier per chunk: while
+// chunk i's softmax and P V run, the scores of chunk i + 1 are formed, chunk i + 2 of K and i + 1 of V are converted
+// into the buffers that became free, and the next raw chunks are on their way into registers. Overflow of the default
+// operand scale is flagged while converting; the flag is read after the barrier that publishes the chunk, and a flagged
+// chunk (outliers) is staged again with its own scale by the whole block.
+//
+// What bounds it: the matrix products (96 instructions of 32 cycles per wave and chunk, one wave per SIMD) and the 80 KB
+// of LDS reads and writes per wave beside them. 32 queries per wave, because every wave reads the whole staged chunk: at
+// 16 queries the LDS reads alone outlast the products; 16 tokens per block halve the K and V read from the caches and
+// the conversions per query. One wave per SIMD hides nothing by itself, hence the hand-placed slices of vector work after each
+// matrix instruction. Registers: accumulators and most of Q in AGPRs (pinned; otherwise the compiler moves all 128
+// accumulators through VGPRs each chunk), no scratch.
+// One 8192-token prompt, 16 heads (550 GFLOP of fp32 products): 3.70 -> 1.67 ms = 329 TFLOP/s (988 of fp16 MFMA issue; a
+// large library bf16 matrix product reaches 1380 on this card). The form before held 16 queries per wave, 8 tokens per
+// block, with P through LDS.
+// AttnPrefill<2> (halo_attn_prefill_d2): 8-token tiles, two waves share 32 queries and split the output dims: 0.75x the
+// matrix work per wave and twice the blocks, for batches whose 8-token tiles fit the 256 CUs once (256 tokens at position
+// 8192: 840 us with 16-token tiles, 734 with these, measured on one build; 1167 before).
+namespace {
+constexpr int kHalf = kChunk * kHd * 2;          // bytes of one staged matrix's hi (or lo) halves
+constexpr int kBuf = 2 * kHalf;                  // bytes of one staged chunk of K or V
+constexpr float kSppT = 1024.0f;                 // probabilities, <= 2^kLazy
+constexpr float kLazy = 5.0f;                    // the running max may lag by this (base 2) before a rescale
+typedef float V16F __attribute__((ext_vector_type(16)));
+typedef short S4 __attribute__((ext_vector_type(4)));
 
-extern "C" __global__ void __launch_bounds__(256, 2) halo_attn_prefill(
+__device__ __forceinline__ V16F Mfma3x32(const H8& ah, const H8& al, const H8& bh, const H8& bl, V16F c) {
+  c = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, c, 0, 0, 0);
+}
+// 4 keys (rows) of one dim (column) per lane: within 16 lanes, lane i addresses 8 bytes of row i / 4 and receives column
+// i of the four rows.
+__device__ __forceinline__ H4 ReadTr(const char* p) {
+  return __builtin_bit_cast(
+      H4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) S4*)(const_cast<char*>(p))));
+}
+// 8 floats of 4 pieces of a K or V row: the largest magnitude, and the conversion of the pieces into a staged row
+__device__ __forceinline__ float MaxAbs(const float4 (&r)[8]) {
+  float a = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) a = fmaxf(a, fmaxf(fmaxf(fabsf(r[e].x), fabsf(r[e].y)), fmaxf(fabsf(r[e].z), fabsf(r[e].w))));
+  return a;
+}
+__device__ __forceinline__ void StagePiece(const float4& u, const float4& v, char* at, float scale) {
+  const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+  H8 hi, lo;
+  SplitHalves(x, hi, lo, scale);
+  *reinterpret_cast<H8*>(at) = hi;
+  *reinterpret_cast<H8*>(at + kHalf) = lo;
+}
+// (piece part + 8 j at byte a0 ^ 128 (j & 1) + 256 (j / 2) of the hi half: the swizzle touches the low four piece bits)
+__device__ __forceinline__ void StageRow(const float4 (&r)[8], char* lds, std::uint32_t a0, float scale) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) StagePiece(r[2 * j], r[2 * j + 1], lds + (a0 ^ (128u * (j & 1))) + 256 * (j / 2), scale);
+}
+}  // namespace
+
+namespace {
+template <int DS>
+__device__ __forceinline__ void AttnPrefill(
     const float* __restrict__ q, const float* __restrict__ gate, const float* __restrict__ kpool,
     const float* __restrict__ vpool, const std::uint32_t* __restrict__ pages, const std::uint32_t* __restrict__ tiles,
     float* __restrict__ o, std::int8_t* __restrict__ oq, float* __restrict__ os, std::uint32_t Hq, std::uint32_t Hkv,
     std::uint32_t max_pages) {
-  __shared__ __attribute__((aligned(16))) _Float16 kh[kChunk * kHd], kl[kChunk * kHd];
-  __shared__ __attribute__((aligned(16))) _Float16 vh[kHd * kChunk], vl[kHd * kChunk];
-  __shared__ __attribute__((aligned(16))) _Float16 ph[4][16 * kChunk], pl[4][16 * kChunk];
-  const std::uint32_t G = Hq / Hkv;
-  const std::uint32_t* tl = tiles + 4 * static_cast<std::size_t>(blockIdx.x);
+  constexpr int NJ = 16 / DS;  // steps of the wave's P V: 8 / DS tiles of 32 dims x two steps of 16 keys
+  // K rows: 16-byte piece c of key at c ^ (key & 15); V rows: at c ^ 2 (key & 7) (four keys of a 16-lane transposing read
+  // in four different 32-byte bank groups)
+  __shared__ __attribute__((aligned(1024))) char lds[4 * kBuf];  // K buffers 0, 1, V buffers 0, 1: hi then lo halves
+  __shared__ float red[4];
+  __shared__ __attribute__((aligned(16))) std::uint32_t flags[2][2][4];  // [buffer][K, V][wave]: default scale overflowed
+  const std::uint32_t* tl = tiles + 4 * static_cast<std::size_t>(blockIdx.x / Hkv);
   const std::uint32_t first = tl[0], ntok = tl[1], sess = tl[2], p0 = tl[3];
-  const std::uint32_t kvh = blockIdx.y;
-  const std::uint32_t t = threadIdx.x, wave = t / kWave, lane = t % kWave;
-  const std::uint32_t row = lane % 16, kq = lane / 16;
-  const std::uint32_t last = p0 + ntok - 1;
-  const std::uint32_t nchunks = last / kChunk + 1;
+  const std::uint32_t kvh = blockIdx.x % Hkv;
+  const std::uint32_t t = threadIdx.x, wave = t / kWave, lane = t % kWave, n = lane % 32, h = lane / 32;
+  const std::uint32_t tok0 = 4 * (wave / DS), d0 = wave % DS * (kHd / DS);  // the wave's first token and output dim
+  const std::uint32_t last = p0 + ntok - 1, nchunks = last / kChunk + 1;
   const std::uint32_t* pt = pages + static_cast<std::size_t>(sess) * max_pages;
-  // staging roles: K rows key = t / 8, 32-byte pieces part + 8 j; V keys 8 (t / 64) + e at dims 4 (t % 64) ..
-  const std::uint32_t skey = t / 8, spart = t % 8, vdg = t % 64, vkg = t / 64;
-  float4 kreg[8], vreg[8];
-  auto load_chunk = [&](std::uint32_t k0) {
-    {
-      const std::uint32_t kp = min(k0 + skey, last);
-      const float4* ks = reinterpret_cast<const float4*>(
-          kpool + ((static_cast<std::size_t>(pt[kp / kPage]) * Hkv + kvh) * kPage + kp % kPage) * kHd);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        kreg[2 * j] = ks[2 * (spart + 8 * j)];
-        kreg[2 * j + 1] = ks[2 * (spart + 8 * j) + 1];
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const std::uint32_t kp = min(k0 + 8 * vkg + e, last);
-      vreg[e] = reinterpret_cast<const float4*>(
-          vpool + ((static_cast<std::size_t>(pt[kp / kPage]) * Hkv + kvh) * kPage + kp % kPage) * kHd)[vdg];
-    }
+  // staging: thread t holds key t / 8 of a chunk, 32-byte pieces part + 8 j
+  const std::uint32_t skey = t / 8, spart = t % 8;
+  const std::uint32_t ksa = skey * 512 + 16 * (spart ^ (skey & 15));
+  const std::uint32_t vsa = 2 * kBuf + skey * 512 + 16 * (spart ^ (2 * (skey & 7)));
+  // reads: K step c (dims 16 c + 8 h ..) of key n at ka ^ 32 (c & 7) + 256 (c / 8); V's keys 4 h + lane % 16 / 4 (+ 8, + 16 per step),
+  // dims 32 c + 16 (lane / 16 % 2) + 4 (lane % 4) at va ^ 64 (c & 3) + 256 (c / 4)
+  const std::uint32_t ka = n * 512 + 16 * (h ^ (n & 15));
+  const std::uint32_t vk = 4 * h + (lane % 16) / 4;
+  const std::uint32_t va = 2 * kBuf + vk * 512 + 16 * ((2 * (lane / 16 % 2) + lane % 4 / 2) ^ (2 * vk)) + 8 * (lane % 2) + 2 * d0;
+  float4 kraw[8], vraw[8];
+  const auto position = [&](std::uint32_t c) { return min(c * kChunk + skey, last); };
+  const auto row = [&](const float* pool, std::uint32_t page, std::uint32_t c) {
+    return reinterpret_cast<const float4*>(
+        pool + ((static_cast<std::size_t>(page) * Hkv + kvh) * kPage + position(c) % kPage) * kHd);
   };
-  auto stage_chunk = [&](float sk, float sv) {
+  const auto load = [&](const float* pool, std::uint32_t page, std::uint32_t c, float4 (&r)[8]) {
+    const float4* s = row(pool, page, c);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float x[8] = {kreg[2 * j].x,     kreg[2 * j].y,     kreg[2 * j].z,     kreg[2 * j].w,
-                          kreg[2 * j + 1].x, kreg[2 * j + 1].y, kreg[2 * j + 1].z, kreg[2 * j + 1].w};
-      H8 hi, lo;
-      SplitHalves(x, hi, lo, sk);
-      const std::uint32_t off = skey * kHd + 8 * ((spart + 8 * j) ^ (skey & 15));
-      *reinterpret_cast<H8*>(&kh[off]) = hi;
-      *reinterpret_cast<H8*>(&kl[off]) = lo;
-    }
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      float x[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = d == 0 ? vreg[e].x : d == 1 ? vreg[e].y : d == 2 ? vreg[e].z : vreg[e].w;
-      H8 hi, lo;
-      SplitHalves(x, hi, lo, sv);
-      const std::uint32_t dim = 4 * vdg + d;
-      const std::uint32_t off = dim * kChunk + 8 * (vkg ^ ((dim >> 2) & 3));
-      *reinterpret_cast<H8*>(&vh[off]) = hi;
-      *reinterpret_cast<H8*>(&vl[off]) = lo;
+      r[2 * j] = s[2 * (spart + 8 * j)];
+      r[2 * j + 1] = s[2 * (spart + 8 * j) + 1];
     }
   };
-  load_chunk(0);
-  // this lane's A-operand query: row r -> token 2 wave + r / 8, head r % 8; dims 32 c + 8 kq .. + 7
-  const std::uint32_t qtok = min(2 * wave + row / 8, ntok - 1), qg = row % 8;
-  const float* qrow = q + ((static_cast<std::size_t>(first) + qtok) * Hq + kvh * G + qg) * kHd;
-  // Operand scales (powers of two, halo::SplitScale): per query row, per chunk for K; V's scale is the smallest of
-  // the chunks so far (the accumulators are rescaled, exactly, when it drops)
-  H8 qh[kHd / 32], ql[kHd / 32];
-  float sqc[4];
+  std::uint32_t pg0 = pt[position(0) / kPage], pg1 = pt[position(1) / kPage], pg2 = pt[position(2) / kPage];
+  // this lane's query: dims 16 c + 8 h .. + 7 of step c (the B operand)
+  const std::uint32_t tok = min(tok0 + n / 8, ntok - 1);
+  const std::size_t qbase = ((static_cast<std::size_t>(first) + tok) * Hq + kvh * 8 + n % 8) * kHd;
+  H8 qh[kHd / 16], ql[kHd / 16];
+  float fq;
   {
-    float xr[kHd / 32][8];
+    const float* qrow = q + qbase + 8 * h;
     float amax = 0.0f;
 #pragma unroll
-    for (int c = 0; c < kHd / 32; ++c) {
-      const float4 a = *reinterpret_cast<const float4*>(qrow + 32 * c + 8 * kq);
-      const float4 b = *reinterpret_cast<const float4*>(qrow + 32 * c + 8 * kq + 4);
-      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        xr[c][e] = x[e];
-        amax = fmaxf(amax, fabsf(x[e]));
-      }
+    for (int c = 0; c < kHd / 16; ++c) {
+      const float4 a = *reinterpret_cast<const float4*>(qrow + 16 * c), b = *reinterpret_cast<const float4*>(qrow + 16 * c + 4);
+      amax = fmaxf(amax, fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
+                               fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w)))));
     }
-    amax = fmaxf(amax, __shfl_xor(amax, 16));
     amax = fmaxf(amax, __shfl_xor(amax, 32));
     const float sq = halo::SplitScale(amax, kSqk);
 #pragma unroll
-    for (int c = 0; c < kHd / 32; ++c) SplitHalves(xr[c], qh[c], ql[c], sq);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sqc[i] = __shfl(sq, 4 * kq + i);  // the scales of this lane's output rows
-  }
-  __shared__ float kvmax[2][4];
-  float sv = kSvv;
-  std::uint32_t qpos[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) qpos[i] = p0 + 2 * wave + (4 * kq + i) / 8;
-  float m[4], l[4];
-  V4F acc[kHd / 16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.0f;
-  }
-#pragma unroll
-  for (int c = 0; c < kHd / 16; ++c) acc[c] = V4F{0.0f, 0.0f, 0.0f, 0.0f};
-  const float scale = 1.0f / sqrtf(static_cast<float>(kHd));
-  _Float16* pwh = &ph[wave][0];
-  _Float16* pwl = &pl[wave][0];
-  for (std::uint32_t ch = 0; ch < nchunks; ++ch) {
-    const std::uint32_t k0 = ch * kChunk;
-    {  // the chunk's K and V magnitudes
-      float ka = 0.0f, va = 0.0f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        ka = fmaxf(ka, fmaxf(fmaxf(fabsf(kreg[e].x), fabsf(kreg[e].y)), fmaxf(fabsf(kreg[e].z), fabsf(kreg[e].w))));
-        va = fmaxf(va, fmaxf(fmaxf(fabsf(vreg[e].x), fabsf(vreg[e].y)), fmaxf(fabsf(vreg[e].z), fabsf(vreg[e].w))));
-      }
-      ka = halo::GroupMax(ka);
-      va = halo::GroupMax(va);
-      if (lane == 0) {
-        kvmax[0][wave] = ka;
-        kvmax[1][wave] = va;
-      }
+    for (int c = 0; c < kHd / 16; ++c) {  // (read again: the row is in the cache, and 128 floats need no registers)
+      const float4 a = *reinterpret_cast<const float4*>(qrow + 16 * c), b = *reinterpret_cast<const float4*>(qrow + 16 * c + 4);
+      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      SplitHalves(x, qh[c], ql[c], sq);
+      __builtin_amdgcn_sched_barrier(0);  // a few of the row's loads at a time
+      asm("" : "+a"(qh[c]));
+      if (c < 8) asm("" : "+a"(ql[c]));
     }
-    __syncthreads();  // every wave is done with the previous chunk's LDS
-    const float sk = halo::SplitScale(fmaxf(fmaxf(kvmax[0][0], kvmax[0][1]), fmaxf(kvmax[0][2], kvmax[0][3])), kSqk);
-    const float svc = halo::SplitScale(fmaxf(fmaxf(kvmax[1][0], kvmax[1][1]), fmaxf(kvmax[1][2], kvmax[1][3])), kSvv);
-    const float vfac = svc < sv ? svc / sv : 1.0f;  // exact: both are powers of two
-    sv = fminf(sv, svc);
-    stage_chunk(sk, sv);
+    // scores and the running max in base-2 units: each exponential is one v_exp_f32
+    fq = (1.0f / sqrtf(static_cast<float>(kHd))) * kLog2e / sq;
+  }
+  load(kpool, pg0, 0, kraw);
+  load(vpool, pg0, 0, vraw);
+  const std::uint32_t qpos = p0 + tok0 + n / 8;
+  float sva = kSvv, ps = kSppT;  // V's scale in acc (the smallest so far), and the scale of P that matches it
+  float m = -INFINITY, l = 0.0f;
+  V16F acc[NJ / 2];
+#pragma unroll
+  for (int c = 0; c < NJ / 2; ++c) {
+    acc[c] = V16F{};
+    asm("" : "+a"(acc[c]));
+  }
+
+  // a chunk of K or V from registers into buffer b at the default scale, flagged by the waves where that overflows (every
+  // lane of a wave stores the same word: a store under a branch would cut the schedule)
+  const auto stage = [&](int which, const float4 (&r)[8], std::uint32_t b) {
+    flags[b ^ which][which][wave] = __any(MaxAbs(r) * 256.0f >= 65504.0f) ? 1u : 0u;
+    StageRow(r, lds, (which ? vsa : ksa) + b * kBuf, 256.0f);
+  };
+  // at iteration i the block reads the pair (K of chunk i + 1, V of chunk i) in one row: K's buffer index and the
+  // complement of V's
+  const auto flagged = [&](std::uint32_t row_) {
+    const uint4 k = *reinterpret_cast<const uint4*>(flags[row_][0]), v = *reinterpret_cast<const uint4*>(flags[row_][1]);
+    const std::uint32_t w = k.x | k.y | k.z | k.w | (v.x | v.y | v.z | v.w) << 1;
+    return __builtin_amdgcn_readfirstlane(w);
+  };
+  static_assert(kSqk == 256.0f && kSvv == 256.0f);
+  // a flagged chunk again, by the whole block, at the scale of its largest magnitude; returns the scale
+  const auto restage = [&](const float* pool, std::uint32_t c, bool is_v, std::uint32_t b, float base) {
+    const float4* src = row(pool, pt[position(c) / kPage], c);
+    float w = 0.0f;
+#pragma unroll 1
+    for (int j = 0; j < 8; ++j) {
+      const float4 x = src[2 * (spart + 8 * (j / 2)) + j % 2];
+      w = fmaxf(w, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
+    }
+    w = halo::GroupMax(w);
+    if (lane == 0) red[wave] = w;
     __syncthreads();
-    if (ch + 1 < nchunks) load_chunk(k0 + kChunk);  // in flight while this chunk computes
-    // scores: two 16 x 16 tiles (keys k0 .. k0 + 15, k0 + 16 .. k0 + 31); B lane (key row, dims 32 c + 8 kq ..)
-    V4F sc[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      V4F c4 = {0.0f, 0.0f, 0.0f, 0.0f};
-      const std::uint32_t key = 16 * h + row;
-#pragma unroll
-      for (int c = 0; c < kHd / 32; ++c) {
-        const std::uint32_t off = key * kHd + 8 * ((4 * c + kq) ^ (key & 15));
-        const H8 bh = *reinterpret_cast<const H8*>(&kh[off]);
-        const H8 bl = *reinterpret_cast<const H8*>(&kl[off]);
-        c4 = Mfma3(qh[c], ql[c], bh, bl, c4);
-      }
-      sc[h] = c4;
+    const float s = halo::SplitScale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])), base);
+    const std::uint32_t a0 = (is_v ? vsa : ksa) + b * kBuf;
+#pragma unroll 1
+    for (int j = 0; j < 4; ++j) {
+      const float4 u = src[2 * (spart + 8 * j)], v = src[2 * (spart + 8 * j) + 1];
+      StagePiece(u, v, lds + (a0 ^ (128u * (j & 1))) + 256 * (j / 2), s);
     }
-    // online softmax per output row (lanes 16 kq .. 16 kq + 15 hold one row's 32 scores)
-    float alpha[4];
-    // Scores and the running max in base-2 units (scale * log2(e) folded into the score scale), so each
-    // exponential is one v_exp_f32 and a masked score (-inf) needs no select.
-    bool rescale = false;
+    __syncthreads();
+    return s;
+  };
+  // operand fragments of K step c and of V step j = 2 c + st (dims 32 c .., keys 16 st ..)
+  const auto kfrag = [&](std::uint32_t b, int c, H8& hi, H8& lo) {
+    const char* at = lds + ((ka + b * kBuf) ^ (32u * (c & 7))) + 256 * (c / 8);
+    hi = *reinterpret_cast<const H8*>(at);
+    lo = *reinterpret_cast<const H8*>(at + kHalf);
+  };
+  const auto vfrag = [&](std::uint32_t b, int j, H8& hi, H8& lo) {
+    const int c = j / 2, st = j % 2;
+    const char* at = lds + ((va + b * kBuf) ^ (64u * (c & 3))) + 256 * (c / 4) + 8192 * st;
+    const H4 h0 = ReadTr(at), h1 = ReadTr(at + 4096), l0 = ReadTr(at + kHalf), l1 = ReadTr(at + kHalf + 4096);
+    hi = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+    lo = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+
+  stage(0, kraw, 0);
+  load(kpool, pg1, 1, kraw);
+  stage(1, vraw, 0);
+  load(vpool, pg1, 1, vraw);
+  __syncthreads();
+  float f = fq / kSqk;
+  if (flagged(0) & 1u) f = fq / restage(kpool, 0, false, 0, kSqk);
+  V16F s = {};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float f = scale * kLog2e / (sqc[i] * sk);
-      float s0 = sc[0][i] * f, s1 = sc[1][i] * f;
-      const std::uint32_t kp0 = k0 + row, kp1 = k0 + 16 + row;
-      s0 = kp0 <= qpos[i] ? s0 : -INFINITY;
-      s1 = kp1 <= qpos[i] ? s1 : -INFINITY;
-      const float cm = halo::GroupMax<16>(fmaxf(s0, s1));
-      const float mx = fmaxf(m[i], cm);
-      const bool none = mx == -INFINITY;
-      alpha[i] = none ? 1.0f : __builtin_amdgcn_exp2f(m[i] - mx);
-      rescale |= alpha[i] != 1.0f;
-      const float e0 = __builtin_amdgcn_exp2f(s0 - mx), e1 = __builtin_amdgcn_exp2f(s1 - mx);
-      l[i] = l[i] * alpha[i] + halo::GroupSum<16>(e0 + e1);
-      m[i] = mx;
-      // P row 4 kq + i, keys row and 16 + row; 16-byte chunk c of a P row at c ^ (kq & 3) (row >> 2 == kq)
-      const std::uint32_t pr = (4 * kq + i) * kChunk;
-      std::uint32_t ph2, pl2;
-      halo::SplitPair(e0, e1, kSpp, ph2, pl2);
-      const std::uint32_t o0 = pr + 8 * ((row / 8) ^ kq) + row % 8, o1 = pr + 8 * ((2 + row / 8) ^ kq) + row % 8;
-      pwh[o0] = __builtin_bit_cast(_Float16, static_cast<std::uint16_t>(ph2 & 0xFFFFu));
-      pwl[o0] = __builtin_bit_cast(_Float16, static_cast<std::uint16_t>(pl2 & 0xFFFFu));
-      pwh[o1] = __builtin_bit_cast(_Float16, static_cast<std::uint16_t>(ph2 >> 16));
-      pwl[o1] = __builtin_bit_cast(_Float16, static_cast<std::uint16_t>(pl2 >> 16));
-    }
-    // the accumulators change only where some row's max moved (rare once the first chunks are in)
-    if (__any(rescale) || vfac != 1.0f)
-#pragma unroll
-      for (int c = 0; c < kHd / 16; ++c)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[c][i] *= alpha[i] * vfac;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // P V: A = P (row = query, k = keys 8 kq ..), B = V (k = keys 8 kq .., col = dim 16 c + row)
-    const std::uint32_t pa = row * kChunk + 8 * (kq ^ ((row >> 2) & 3));
-    const H8 pah = *reinterpret_cast<const H8*>(&pwh[pa]);
-    const H8 pal = *reinterpret_cast<const H8*>(&pwl[pa]);
-#pragma unroll
-    for (int c = 0; c < kHd / 16; ++c) {
-      const std::uint32_t dim = 16 * c + row;
-      const std::uint32_t off = dim * kChunk + 8 * (kq ^ ((dim >> 2) & 3));
-      const H8 bh = *reinterpret_cast<const H8*>(&vh[off]);
-      const H8 bl = *reinterpret_cast<const H8*>(&vl[off]);
-      acc[c] = Mfma3(pah, pal, bh, bl, acc[c]);
-    }
+  for (int c = 0; c < kHd / 16; ++c) {
+    H8 ah, al;
+    kfrag(0, c, ah, al);
+    s = Mfma3x32(ah, al, qh[c], ql[c], s);
   }
-  // epilogue: rows 4 kq + i, dims 16 c + row
+  // masked scores of a chunk (slot j: key 8 (j / 4) + 4 h + j % 4 of it; lim: the query's position in it, less 4 h) and
+  // their largest over the lane pair
+  const auto mask = [&](float x, int j, int lim) { return 8 * (j / 4) + j % 4 <= lim ? x : -INFINITY; };
+  const auto pair_max = [](float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  };
+  float cm = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const std::uint32_t r = 4 * kq + i;
-    const std::uint32_t tok = 2 * wave + r / 8, g = r % 8;
-    const bool live = tok < ntok;
-    const std::size_t base = ((static_cast<std::size_t>(first) + min(tok, ntok - 1)) * Hq + kvh * G + g) * kHd;
-    const float inv = 1.0f / l[i] * (1.0f / (kSpp * sv));
+  for (int j = 0; j < 16; ++j) {
+    s[j] = mask(s[j], j, static_cast<int>(qpos - 4 * h));
+    cm = fmaxf(cm, s[j]);
+  }
+  cm = pair_max(cm) * f;
+  stage(0, kraw, 1);
+  load(kpool, pg2, 2, kraw);
+  pg1 = pg2;  // at iteration i: pg1, pg2 the pages of chunks i + 2, i + 3
+  pg2 = pt[position(3) / kPage];
+  for (std::uint32_t i = 0; i < nchunks; ++i) {
+    const std::uint32_t b = i & 1, nb = b ^ 1;
+    halo::LdsSync();  // K of chunk i + 1 and V of chunk i are staged; the buffers of K i and V i - 1 are free
+    float fn = fq / kSqk, vfac = 1.0f;  // score factor of chunk i + 1 (exact: the scales are powers of two)
+    const std::uint32_t fl = flagged(nb);
+    if (fl != 0u) {
+      if (fl & 1u) fn = fq / restage(kpool, i + 1, false, nb, kSqk);
+      const float svc = fl & 2u ? restage(vpool, i, true, b, kSvv) : kSvv;
+      vfac = svc < sva ? svc / sva : 1.0f;
+      sva = fminf(sva, svc);
+      ps = kSppT * (sva / svc);
+    } else {
+      ps = kSppT * (sva / kSvv);
+    }
+    // the running max (base-2 units) lags by up to kLazy, so few chunks rescale
+    if (__any(cm > m + kLazy) || vfac != 1.0f) {
+      const float mx = fmaxf(m, cm);
+      const float alpha = mx == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mx);
+      m = mx;
+      l *= alpha;
 #pragma unroll
-    for (int c = 0; c < kHd / 16; c += 2) {
-      const std::uint32_t d0 = 16 * c + row, d1 = 16 * (c + 1) + row;
-      const float v0 = acc[c][i] * inv * halo::Sigmoid(gate[base + d0]);
-      const float v1 = acc[c + 1][i] * inv * halo::Sigmoid(gate[base + d1]);
-      if (live && o != nullptr) {
-        o[base + d0] = v0;
-        o[base + d1] = v1;
+      for (int c = 0; c < NJ / 2; ++c) {
+        // through vector registers 16 at a time: without the pins the accumulators live there from the loop's start on,
+        // and every iteration copies all of them
+        V16F a = acc[c];
+        asm("" : "+v"(a));
+        a *= alpha * vfac;
+        asm("" : "+a"(a));
+        acc[c] = a;
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (oq != nullptr) {
-        const float amax = halo::GroupMax<16>(fmaxf(fabsf(v0), fabsf(v1)));
-        const float qs = amax / 127.0f;
-        if (live) {
-          oq[base + d0] = static_cast<std::int8_t>(qs > 0.0f ? static_cast<int>(rintf(v0 / qs)) : 0);
-          oq[base + d1] = static_cast<std::int8_t>(qs > 0.0f ? static_cast<int>(rintf(v1 / qs)) : 0);
-          if (row == 0) os[(base + 16 * c) / 32] = qs;
+    }
+    // P^T of chunk i (slots 8 st .. 8 st + 7 are the k order of step st) beside the scores of chunk i + 1 (past the end:
+    // the clamped chunk's, unused), then P V beside the conversions: after each matrix instruction a slice of the vector
+    // work that it hides (the barriers keep that order), each step's fragments read one step ahead.
+    H8 ah[2], al[2];
+    V16F sn = {};
+    float e[16], ls = 0.0f;
+    std::uint32_t pw[16], sw[8];
+    const auto softmax_slice = [&](int k) {  // k < 24: scores 2 p, 2 p + 1 in slices 3 p .. 3 p + 2
+      const int p = k / 3;
+      if (k >= 24) return;
+      if (k % 3 == 0) {
+        e[2 * p] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * p], f, -m));
+        e[2 * p + 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * p + 1], f, -m));
+      } else if (k % 3 == 1) {
+        halo::SplitPair(e[2 * p], e[2 * p + 1], ps, pw[p], pw[8 + p]);
+      } else {
+        ls += e[2 * p] + e[2 * p + 1];
+      }
+    };
+    // k < 24: as stage(which, buf), in four pieces: its splits, its two stores, and the same piece of the chunk after into
+    // the registers that became free (in flight for a whole iteration)
+    const auto stage_slice = [&](int k, int which, float4 (&r)[8], const float4* next, std::uint32_t buf, float& top) {
+      const int j = k / 6, e = k % 6;
+      if (e < 4) {
+        const float4 x = r[2 * j + e / 2];
+        halo::SplitPair(e % 2 ? x.z : x.x, e % 2 ? x.w : x.y, 256.0f, sw[e], sw[4 + e]);
+        if (e % 2 == 0) top = fmaxf(top, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
+      } else if (e == 4) {
+        char* at = lds + (((which ? vsa : ksa) + buf * kBuf) ^ (128u * (j & 1))) + 256 * (j / 2);
+        *reinterpret_cast<uint4*>(at) = make_uint4(sw[0], sw[1], sw[2], sw[3]);
+        *reinterpret_cast<uint4*>(at + kHalf) = make_uint4(sw[4], sw[5], sw[6], sw[7]);
+      } else {
+        r[2 * j] = next[2 * (spart + 8 * j)];
+        r[2 * j + 1] = next[2 * (spart + 8 * j) + 1];
+        if (j == 3) flags[buf ^ which][which][wave] = __any(top * 256.0f >= 65504.0f) ? 1u : 0u;
+      }
+    };
+    // k < 24: the masked scores of chunk i + 1 and their max (from slice 4 on: the last score product has landed)
+    const int lim = static_cast<int>(qpos - 4 * h) - static_cast<int>(i * kChunk + kChunk);
+    const auto score_slice = [&](int k) {
+      if (k >= 4 && k < 20) {
+        s[k - 4] = mask(sn[k - 4], k - 4, lim);
+        cm = fmaxf(cm, s[k - 4]);
+      } else if (k == 20) {
+        cm = pair_max(cm) * fn;
+      }
+    };
+    const float4 *knext = nullptr, *vnext = nullptr;
+    kfrag(nb, 0, ah[0], al[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) softmax_slice(k);  // while the first fragments arrive
+    __builtin_amdgcn_sched_barrier(0);
+    float top = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      if (c < 15)
+        kfrag(nb, c + 1, ah[(c + 1) % 2], al[(c + 1) % 2]);
+      else
+        vfrag(b, 0, ah[0], al[0]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(p == 0 ? al[c % 2] : ah[c % 2], p == 1 ? ql[c] : qh[c], sn, 0, 0, 0);
+        if (c == 0 && p == 1) {
+          knext = row(kpool, pg2, i + 3);
+          vnext = row(vpool, pg1, i + 2);
+          pg1 = pg2;
+          pg2 = pt[position(i + 4) / kPage];  // ahead of this iteration's row loads: not waited for with them
         }
+        if (c < 8)
+          softmax_slice(3 * c + p + 9 < 24 ? 3 * c + p + 9 : 24);
+        else
+          stage_slice(3 * (c - 8) + p, 0, kraw, knext, b, top);
+        __builtin_amdgcn_sched_barrier(0);
       }
+    }
+    l += ls;
+    cm = -INFINITY;
+    H8 ph[2], pl[2];
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      ph[st] = __builtin_bit_cast(H8, make_uint4(pw[4 * st], pw[4 * st + 1], pw[4 * st + 2], pw[4 * st + 3]));
+      pl[st] = __builtin_bit_cast(H8, make_uint4(pw[8 + 4 * st], pw[9 + 4 * st], pw[10 + 4 * st], pw[11 + 4 * st]));
+    }
+    top = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (j < NJ - 1) vfrag(b, j + 1, ah[(j + 1) % 2], al[(j + 1) % 2]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        acc[j / 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(p == 0 ? al[j % 2] : ah[j % 2], p == 1 ? pl[j % 2] : ph[j % 2],
+                                                             acc[j / 2], 0, 0, 0);
+        if (j < 8) score_slice(3 * j + p);
+        if (j >= NJ - 8) stage_slice(3 * (j - (NJ - 8)) + p, 1, vraw, vnext, nb, top);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    f = fn;
+  }
+  // epilogue: this lane's query, dims d0 + 32 c + 8 g + 4 h + e (slot 4 g + e)
+  l += __shfl_xor(l, 32);
+  const bool live = tok0 + n / 8 < ntok;
+  const float inv = 1.0f / l * (1.0f / (kSppT * sva));
+#pragma unroll
+  for (int c = 0; c < NJ / 2; ++c) {
+    float v[16], amax = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const std::size_t at = qbase + d0 + 32 * c + 8 * g + 4 * h;
+      const float4 gt = *reinterpret_cast<const float4*>(gate + at);
+      v[4 * g] = acc[c][4 * g] * inv * halo::Sigmoid(gt.x);
+      v[4 * g + 1] = acc[c][4 * g + 1] * inv * halo::Sigmoid(gt.y);
+      v[4 * g + 2] = acc[c][4 * g + 2] * inv * halo::Sigmoid(gt.z);
+      v[4 * g + 3] = acc[c][4 * g + 3] * inv * halo::Sigmoid(gt.w);
+      if (live && o != nullptr) *reinterpret_cast<float4*>(o + at) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(v[4 * g + e]));
+    }
+    if (oq != nullptr) {  // a Q8 block is this step's 32 dims: 16 in each lane of the pair
+      const float qs = fmaxf(amax, __shfl_xor(amax, 32)) / 127.0f;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        std::uint32_t word = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int code = qs > 0.0f ? static_cast<int>(rintf(v[4 * g + e] / qs)) : 0;
+          word |= (static_cast<std::uint32_t>(code) & 0xFFu) << (8 * e);
+        }
+        if (live) *reinterpret_cast<std::uint32_t*>(oq + qbase + d0 + 32 * c + 8 * g + 4 * h) = word;
+      }
+      if (live && h == 0) os[(qbase + d0 + 32 * c) / 32] = qs;
     }
   }
 }
+}  // namespace
+
+#define HALO_ATTN_PREFILL(NAME, DS)                                                                                   \
+  extern "C" __global__ void __launch_bounds__(256, 1) NAME(                                                          \
+      const float* q, const float* gate, const float* kpool, const float* vpool, const std::uint32_t* pages,          \
+      const std::uint32_t* tiles, float* o, std::int8_t* oq, float* os, std::uint32_t Hq, std::uint32_t Hkv,          \
+      std::uint32_t max_pages) {                                                                                      \
+    AttnPrefill<DS>(q, gate, kpool, vpool, pages, tiles, o, oq, os, Hq, Hkv, max_pages);                              \
+  }
+HALO_ATTN_PREFILL(halo_attn_prefill, 1)
+HALO_ATTN_PREFILL(halo_attn_prefill_d2, 2)
+#undef HALO_ATTN_PREFILL

@@ -88,3 +88,45 @@ def run_case(dev, S, prefix, segs, max_context, qk=1.0, v=1.0, abs_tol=1e-6, out
     xq, xs = O.quantize(got.reshape(T, Hq * D))
     assert np.array_equal(goq.download(), xq)
     assert np.array_equal(gos.download().view(np.uint32), xs.view(np.uint32))
+
+
+@pytest.mark.parametrize("segs", [
+    [(0, 0, 7), (0, 7, 1), (0, 8, 8), (0, 16, 9)],  # 8-token tiles: below, at and past one
+    [(0, 0, 33)],
+])
+def test_attn_prefill_tile_edges(dev, segs):
+    run_case(dev, 1, 0, segs, 64)
+
+
+def test_attn_prefill_tile_shapes_bitwise(dev):
+    """A 1100-token prompt takes 16-token tiles, the same prompt in calls of 512 tokens 8-token ones (the output dims split
+    over two waves): a query's operations are the same in both, so the outputs are equal bit for bit; and tokens at
+    the edges of tiles and chunks match softmax attention in 64 bits within 1e-5 of sum |p| |v|."""
+    Hq, Hkv, T = 16, 2, 1100
+    rng = np.random.default_rng(11)
+    desc, g, kp, vp, pages, _ = build(dev, rng, 1, Hkv, 0, [1104], 1104, 2.0, 1.0)
+    q = (2.0 * rng.normal(0, 1, (T, Hq, D))).astype(np.float32)
+    gate = rng.normal(0, 1, (T, Hq, D)).astype(np.float32)
+    gq, gg = dev.to_device(q), dev.to_device(gate)
+
+    def run(pieces):
+        go = dev.array((T, Hq, D), np.float32).fill(0)
+        for start, n in pieces:
+            seg = (H.PrefillSegment * 1)(H.PrefillSegment(0, start, n, start))
+            nbytes = H.lib().halo_op_attn_prefill_workspace_bytes(seg, 1)
+            ws = dev.array(nbytes, np.uint8)
+            dev.op("attn_prefill", ctypes.byref(desc), seg, 1, gq.ptr, gg.ptr, go.ptr, None, None, Hq, ws.ptr, nbytes)
+            dev.sync()
+        return go.download()
+
+    whole = run([(0, T)])
+    assert np.array_equal(whole.view(np.uint32), run([(0, 512), (512, 512), (1024, 76)]).view(np.uint32))
+    for p in (0, 3, 15, 16, 31, 32, 33, 511, 1087, 1088, T - 1):
+        for h in (0, 7, 8, 15):
+            K = gather(kp, pages[0], p + 1, h // 8).astype(np.float64)
+            V = gather(vp, pages[0], p + 1, h // 8).astype(np.float64)
+            s = K @ q[p, h].astype(np.float64) / 16.0
+            pr = np.exp(s - s.max())
+            pr /= pr.sum()
+            sg = 1 / (1 + np.exp(-gate[p, h].astype(np.float64)))
+            assert np.all(np.abs(whole[p, h] - pr @ V * sg) <= 1e-5 * (pr @ np.abs(V)) * sg + 1e-7), f"token {p} head {h}"
