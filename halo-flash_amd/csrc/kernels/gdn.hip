@@ -103,7 +103,7 @@ extern "C" __global__ void __launch_bounds__(256)
 // zero. Inputs q, k [tokens][Hk][128] and v [tokens][Hv][128] are bf16 (the C3 operator) or fp32 (the model's
 // prefill, which matches its decode step); g, beta [tokens][Hv] fp32 (g = log decay, beta after its sigmoid); state
 // fp32 [seq][Hv][128][128] key-major. chunks [n][3] = {first token, length, sequence}; seqs [n_seq][2] = {first
-// chunk, chunk count}. Workspace per (chunk, head): Uk, Qe, Wv, Ov fp32 [64][128] and G [64].
+// chunk, chunk count}. Workspace per (chunk, head): Uk, Qe, Wv, Ov fp32 [64][128] and the weights [64].
 namespace {
 constexpr int kC = 64;
 constexpr int kCL = 132;  // LDS row stride (floats) of a 64 x 128 tile
@@ -134,197 +134,258 @@ __device__ __forceinline__ void Put8(float* dst, const Pack8<In>& x, bool on) {
 }
 }  // namespace
 
-// grid (n_chunks, Hv), block 512 (8 waves). MFMA v_mfma_f32_32x32x2f32: A lane l = A[l % 32][k], B lane l =
-// B[k][l % 32] with k split in halves (lanes 0-31 the first half of the K range, 32-63 the second), D lane l holds
-// column l % 32 and rows 8 (r / 4) + 4 (l / 32) + r % 4. Wave w owns the 32 x 32 tile ((w % 4) / 2, w % 2) of K K^T
-// (w < 4) or Q K^T (w >= 4), then the 32-column tile 2 (w % 2) + w / 4 of each 64 x 128 product. T = (I + A)^-1 by
-// forward substitution in wave 0, one column per lane, in registers.
+// grid (n_chunks, Hv), block 512 (8 waves). All products on v_mfma_f32_16x16x4f32 with instruction e of a 16-deep step taking
+// k = 4 (lane / 16) + e: an A operand is then 16 bytes of a row, and a result (column lane % 16, rows 4 (lane / 16) + r) is in
+// place the B operand of a product over its rows. A (then T = (I + A)^-1) and P are lower triangular: the ten 16 x 16
+// tiles on and below the diagonal, tile i (i + 1) / 2 + j in LDS with rows of 20 floats (free of bank conflicts), and
+// nothing above is computed.
+//   1. K into LDS (fp32, 16-byte groups xor-swizzled by the row); the 20 tiles of K K^T and Q K^T over the waves (five per
+//      SIMD), Q rows straight from memory; scaled into A and P.
+//   2. T by 16 x 16 blocks: four waves invert the diagonal blocks by forward substitution (a column per lane), then each
+//      forms one block column, T_ij = -T_ii sum_m A_im T_mj, its blocks passing from result to operand in registers.
+//   3. wave w, columns 16 w .. + 16: Uk = (T diag(beta gamma)) K and Wv = (T diag(beta)) V, and from those registers
+//      Qe = diag(gamma) Q - P Uk and Ov = P Wv.
+// What bounds it: the fp32 matrix products (80 + 160 + 160 instructions of 32 cycles per SIMD pair of waves); 59 KB of LDS,
+// so that two blocks per CU cover each other's barriers and the substitution. (With whole 64 x 64 products, K, Q and V
+// in 137 KB of LDS and the substitution in one wave: 0.76 ms on the ragged batch {37, 512, 2048, 8191}; this 0.37 ms, of
+// which the 709 MB it writes take about half.)
+namespace {
+constexpr int kTS = 20;          // floats per row of a 16 x 16 tile
+constexpr int kTF = 16 * kTS;    // floats per tile
+__device__ __forceinline__ constexpr int Tri(int i, int j) { return i * (i + 1) / 2 + j; }
+__device__ __forceinline__ V4F Mfma16(const float4& a, const V4F& b, V4F c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[0], c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[1], c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[2], c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[3], c, 0, 0, 0);
+}
+__device__ __forceinline__ float4 Ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 Ld4(const std::uint16_t* p) {
+  const ushort4 u = *reinterpret_cast<const ushort4*>(p);
+  return make_float4(Bf(u.x), Bf(u.y), Bf(u.z), Bf(u.w));
+}
+
 template <typename In>
 __device__ __forceinline__ void WyPrep(const In* __restrict__ q, const In* __restrict__ k, const In* __restrict__ v,
                                        const float* __restrict__ g, const float* __restrict__ beta,
                                        const std::uint32_t* __restrict__ chunks, float* __restrict__ wy,
-                                       float* __restrict__ Gc, std::uint32_t Hv, std::uint32_t Hk) {
-  __shared__ __attribute__((aligned(16))) float kl[kC][kCL];
-  __shared__ __attribute__((aligned(16))) float ql[kC][kCL];
-  __shared__ __attribute__((aligned(16))) float vl[kC][kCL];
-  __shared__ __attribute__((aligned(16))) float am[kC][kPL];  // A, then T
-  __shared__ __attribute__((aligned(16))) float pm[kC][kPL];
-  __shared__ float G[kC], Bt[kC], Bg[kC], Gm[kC];
+                                       float* __restrict__ Wt, std::uint32_t Hv, std::uint32_t Hk) {
+  __shared__ __attribute__((aligned(16))) float kl[kC * kD];
+  __shared__ __attribute__((aligned(16))) float am[10 * kTF], pm[10 * kTF];
+  __shared__ __attribute__((aligned(16))) float G[kC], Gl[kC], Bt[kC], Bg[kC], Gm[kC];  // G + Gl: the log-decays
   const std::uint32_t c = blockIdx.x, h = blockIdx.y, kh = h % Hk, tid = threadIdx.x;
-  const std::uint32_t wave = tid / kWave, lane = tid % kWave, fr = lane % 32, hh = lane / 32;
+  const std::uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave, fc = lane % 16, fq = lane / 16;
   const std::uint32_t start = chunks[c * 3], L = chunks[c * 3 + 1];
-  for (std::uint32_t idx = tid; idx < kC * (kD / 8); idx += blockDim.x) {
-    const std::uint32_t t = idx / (kD / 8), p = idx % (kD / 8), tt = min(t, L - 1);
-    const bool on = t < L;
-    const std::size_t kq = (static_cast<std::size_t>(start + tt) * Hk + kh) * kD + p * 8;
-    const std::size_t vv = (static_cast<std::size_t>(start + tt) * Hv + h) * kD + p * 8;
-    Put8(&kl[t][p * 8], Ld8(k + kq), on);
-    Put8(&ql[t][p * 8], Ld8(q + kq), on);
-    Put8(&vl[t][p * 8], Ld8(v + vv), on);
+  const auto klat = [&](std::uint32_t t, std::uint32_t f4) { return &kl[t * kD + 4 * (f4 ^ (t & 7))]; };
+  const In* kbase = k + (static_cast<std::size_t>(start) * Hk + kh) * kD;
+  const In* qbase = q + (static_cast<std::size_t>(start) * Hk + kh) * kD;
+  const In* vbase = v + (static_cast<std::size_t>(start) * Hv + h) * kD;
+  // K: thread -> rows tid / 16 and + 32, 8 values at 8 (tid % 16)
+  const std::uint32_t kt = tid / 16, kp = tid % 16;
+  const Pack8<In> k0 = Ld8(kbase + static_cast<std::size_t>(min(kt, L - 1)) * Hk * kD + 8 * kp);
+  const Pack8<In> k1 = Ld8(kbase + static_cast<std::size_t>(min(kt + 32, L - 1)) * Hk * kD + 8 * kp);
+  float gv = 0.0f, bv = 0.0f;
+  if (wave == 0) {
+    const std::size_t at = static_cast<std::size_t>(start + min(lane, L - 1)) * Hv + h;
+    gv = lane < L ? g[at] : 0.0f;
+    bv = lane < L ? beta[at] : 0.0f;
   }
-  if (tid < kC) {
-    const std::uint32_t tt = min(tid, L - 1);
-    const bool on = tid < L;
-    const float gv = g[static_cast<std::size_t>(start + tt) * Hv + h], bv = beta[static_cast<std::size_t>(start + tt) * Hv + h];
-    G[tid] = on ? gv : 0.0f;
-    Bt[tid] = on ? bv : 0.0f;
+  const auto put = [&](std::uint32_t t, const Pack8<In>& x) {
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = t < L ? Cv(x.v[e]) : 0.0f;
+    *reinterpret_cast<float4*>(klat(t, 2 * kp)) = make_float4(f[0], f[1], f[2], f[3]);
+    *reinterpret_cast<float4*>(klat(t, 2 * kp + 1)) = make_float4(f[4], f[5], f[6], f[7]);
+  };
+  put(kt, k0);
+  put(kt + 32, k1);
+  if (wave == 0) {  // cumulative log-decays, in double: tokens apart by little are weighted by differences of large sums
+    double sum = gv;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const double up = __shfl_up(sum, d);
+      sum += lane >= static_cast<std::uint32_t>(d) ? up : 0.0;
+    }
+    const float hi = static_cast<float>(sum), lo = static_cast<float>(sum - hi);
+    const float e = expf(hi), gm = __builtin_fmaf(e, lo, e);
+    G[lane] = hi;
+    Gl[lane] = lo;
+    Bt[lane] = bv;
+    Gm[lane] = gm;
+    Bg[lane] = bv * gm;
   }
   __syncthreads();
-  if (tid == 0) {  // running sum in a register: the loads are independent, only the adds form a chain
-    float run = G[0];
+  // tiles of K K^T (jobs 0-9) and Q K^T (10-19)
 #pragma unroll
-    for (int t = 1; t < kC; ++t) {
-      run += G[t];
-      G[t] = run;
+  for (int n = 0; n < 3; ++n) {
+    const std::uint32_t job = wave + 8 * n;
+    if (job < 20) {
+      const bool isp = job >= 10;
+      const std::uint32_t tl = isp ? job - 10 : job, i = tl < 1 ? 0 : tl < 3 ? 1 : tl < 6 ? 2 : 3, j = tl - i * (i + 1) / 2;
+      const std::uint32_t ra = 16 * i + fc, rb = 16 * j + fc;
+      float4 a[8];
+      if (isp) {
+        const In* qr = qbase + static_cast<std::size_t>(min(ra, L - 1)) * Hk * kD + 4 * fq;
+#pragma unroll
+        for (int sb = 0; sb < 8; ++sb) a[sb] = Ld4(qr + 16 * sb);
+      } else {
+#pragma unroll
+        for (int sb = 0; sb < 8; ++sb) a[sb] = *reinterpret_cast<const float4*>(klat(ra, 4 * sb + fq));
+      }
+      V4F acc[2] = {V4F{0.0f, 0.0f, 0.0f, 0.0f}, V4F{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+      for (int sb = 0; sb < 8; ++sb)
+        acc[sb % 2] = Mfma16(a[sb], __builtin_bit_cast(V4F, *reinterpret_cast<const float4*>(klat(rb, 4 * sb + fq))), acc[sb % 2]);
+      const float4 gt = *reinterpret_cast<const float4*>(&G[16 * i + 4 * fq]), bt = *reinterpret_cast<const float4*>(&Bt[16 * i + 4 * fq]);
+      const float4 gl = *reinterpret_cast<const float4*>(&Gl[16 * i + 4 * fq]);
+      const float gs = G[rb], gsl = Gl[rb], gta[4] = {gt.x, gt.y, gt.z, gt.w}, gla[4] = {gl.x, gl.y, gl.z, gl.w};
+      const float bta[4] = {bt.x, bt.y, bt.z, bt.w};
+      float* out = (isp ? pm : am) + tl * kTF + 4 * fq * kTS + fc;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const std::uint32_t t = 16 * i + 4 * fq + r;
+        const float x = acc[0][r] + acc[1][r], dec = expf(rb <= t ? (gta[r] - gs) + (gla[r] - gsl) : 0.0f);
+        out[r * kTS] = isp ? (rb <= t ? dec * x : 0.0f) : (rb < t ? bta[r] * dec * x : 0.0f);
+      }
     }
   }
-  __syncthreads();
-  if (tid < kC) {
-    Gm[tid] = expf(G[tid]);
-    Bg[tid] = Bt[tid] * expf(G[tid]);
-  }
-  // K K^T (waves 0-3) and Q K^T (waves 4-7), tile (ti, tj) = ((wave % 4) / 2, wave % 2), K range = 128 keys
-  // (step s: key s + 64 hh); eight waves, two per SIMD, so one wave's MFMA chain overlaps another's loads and stores
-  const std::uint32_t w4 = wave % 4, ti = w4 / 2, tj = w4 % 2, half = wave / 4;
-  float(*xa)[kCL] = half ? ql : kl;
-  V16F kq = {};
-#pragma unroll 4
-  for (int sb = 0; sb < 16; ++sb) {
-    const float4 xa4 = *reinterpret_cast<const float4*>(&xa[32 * ti + fr][4 * sb + 64 * hh]);
-    const float4 kb = *reinterpret_cast<const float4*>(&kl[32 * tj + fr][4 * sb + 64 * hh]);
-    kq = __builtin_amdgcn_mfma_f32_32x32x2f32(xa4.x, kb.x, kq, 0, 0, 0);
-    kq = __builtin_amdgcn_mfma_f32_32x32x2f32(xa4.y, kb.y, kq, 0, 0, 0);
-    kq = __builtin_amdgcn_mfma_f32_32x32x2f32(xa4.z, kb.z, kq, 0, 0, 0);
-    kq = __builtin_amdgcn_mfma_f32_32x32x2f32(xa4.w, kb.w, kq, 0, 0, 0);
-  }
-  __syncthreads();  // Gm / Bg visible
+  // this wave's columns of V (B operand) and Q (result layout), in flight across the inversion
+  const std::uint32_t col = 16 * wave + fc;
+  V4F vb[4], qc[4];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const std::uint32_t t = 32 * ti + 8 * (r / 4) + 4 * hh + r % 4, s = 32 * tj + fr;
-    const bool low = s < t, leq = s <= t;
-    const float dec = expf(leq ? G[t] - G[s] : 0.0f);
-    if (half)
-      pm[t][s] = leq ? dec * kq[r] : 0.0f;
-    else
-      am[t][s] = low ? Bt[t] * dec * kq[r] : 0.0f;
-  }
-  __syncthreads();
-  // T = (I + A)^-1: lane = column, rows in order; A rows are read as broadcasts, four partial sums per row
-  if (wave == 0) {
-    float T[kC];
+  for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int t = 0; t < kC; ++t) {
-      float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int e = 0; e < 4; ++e) {
+      const std::size_t t = min(16u * m + 4 * fq + e, L - 1);
+      vb[m][e] = Cv(vbase[t * Hv * kD + col]);
+      qc[m][e] = Cv(qbase[t * Hk * kD + col]);
+    }
+  halo::LdsSync();
+  if (wave < 4) {  // diagonal block `wave`
+    float* d = am + Tri(wave, wave) * kTF;
+    float T[16];
 #pragma unroll
-      for (int s4 = 0; s4 < t; s4 += 4) {
-        const float4 ar = *reinterpret_cast<const float4*>(&am[t][s4]);
+    for (int t = 0; t < 16; ++t) {
+      float s4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int x = 0; x < t; x += 4) {
+        const float4 ar = *reinterpret_cast<const float4*>(d + t * kTS + x);
         const float av[4] = {ar.x, ar.y, ar.z, ar.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (s4 + e < t) acc[e] = __builtin_fmaf(av[e], T[s4 + e], acc[e]);
+          if (x + e < t) s4[e] = __builtin_fmaf(av[e], T[x + e], s4[e]);
       }
-      const float sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-      T[t] = lane == static_cast<std::uint32_t>(t) ? 1.0f : -sum;
+      T[t] = (fc == static_cast<std::uint32_t>(t) ? 1.0f : 0.0f) - ((s4[0] + s4[1]) + (s4[2] + s4[3]));
     }
-    // every lane has read all of A above (program order within the wave); T replaces it
 #pragma unroll
-    for (int t = 0; t < kC; ++t) am[t][lane] = T[t];
+    for (int t = 0; t < 16; ++t) d[t * kTS + fc] = T[t];  // (the block's rows have all been read: program order)
   }
-  __syncthreads();
-  // Uk = T diag(beta gamma) K and Wv = T diag(beta) V: wave w owns rows 32 ti, columns 32 (2 (w % 2) + w / 4);
-  // K range = 64 tokens (step s: token s + 32 hh)
+  halo::LdsSync();
+  const auto atile = [&](const float* m, int tl) { return *reinterpret_cast<const float4*>(m + tl * kTF + fc * kTS + 4 * fq); };
+  V4F tc[4];
+  if (wave < 4) {  // block column `wave` of T
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (static_cast<std::uint32_t>(j) == wave) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tc[j][e] = am[Tri(j, j) * kTF + (4 * fq + e) * kTS + fc];
+#pragma unroll
+        for (int i = j + 1; i < 4; ++i) {
+          V4F acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int m = j; m < i; ++m) acc = Mfma16(atile(am, Tri(i, m)), tc[m], acc);
+          const V4F z = {0.0f, 0.0f, 0.0f, 0.0f};
+          tc[i] = -Mfma16(atile(am, Tri(i, i)), acc, z);
+        }
+      }
+  }
+  halo::LdsSync();  // A has been read
+  if (wave < 4) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (static_cast<std::uint32_t>(j) == wave) {
+#pragma unroll
+        for (int i = j + 1; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) am[Tri(i, j) * kTF + (4 * fq + e) * kTS + fc] = tc[i][e];
+      }
+  }
+  halo::LdsSync();
+  V4F uk[4], wv[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) uk[i] = wv[i] = V4F{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    V4F kb;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const std::uint32_t t = 16 * m + 4 * fq + e;
+      kb[e] = klat(t, col / 4)[col % 4];
+    }
+    const float4 bg = *reinterpret_cast<const float4*>(&Bg[16 * m + 4 * fq]), bt = *reinterpret_cast<const float4*>(&Bt[16 * m + 4 * fq]);
+#pragma unroll
+    for (int i = m; i < 4; ++i) {
+      const float4 t = atile(am, Tri(i, m));
+      uk[i] = Mfma16(make_float4(t.x * bg.x, t.y * bg.y, t.z * bg.z, t.w * bg.w), kb, uk[i]);
+      wv[i] = Mfma16(make_float4(t.x * bt.x, t.y * bt.y, t.z * bt.z, t.w * bt.w), vb[m], wv[i]);
+    }
+  }
   float* out = wy + (static_cast<std::size_t>(c) * Hv + h) * 4 * kC * kD;  // Uk, Qe, Wv, Ov
-  const std::uint32_t col = 32 * (2 * tj + half) + fr;
-  V16F uk = {}, wv = {};
-#pragma unroll 2
-  for (int sb = 0; sb < 8; ++sb) {
-    const float4 ta = *reinterpret_cast<const float4*>(&am[32 * ti + fr][4 * sb + 32 * hh]);
-    const float tv[4] = {ta.x, ta.y, ta.z, ta.w};
+  const auto store = [&](int which, int i, const V4F& x) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const std::uint32_t tok = 4 * sb + e + 32 * hh;
-      uk = __builtin_amdgcn_mfma_f32_32x32x2f32(tv[e], Bg[tok] * kl[tok][col], uk, 0, 0, 0);
-      wv = __builtin_amdgcn_mfma_f32_32x32x2f32(tv[e], Bt[tok] * vl[tok][col], wv, 0, 0, 0);
+    for (int r = 0; r < 4; ++r) out[which * kC * kD + (16 * i + 4 * fq + r) * kD + col] = x[r];
+  };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    store(0, i, uk[i]);
+    store(2, i, wv[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 gm = *reinterpret_cast<const float4*>(&Gm[16 * i + 4 * fq]);
+    V4F qe = {gm.x * qc[i][0], gm.y * qc[i][1], gm.z * qc[i][2], gm.w * qc[i][3]}, ov = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int m = 0; m <= i; ++m) {
+      const float4 p = atile(pm, Tri(i, m));
+      qe = Mfma16(make_float4(-p.x, -p.y, -p.z, -p.w), uk[m], qe);
+      ov = Mfma16(p, wv[m], ov);
     }
+    store(1, i, qe);
+    store(3, i, ov);
   }
-  __syncthreads();  // K and V are no longer read: Uk and Wv take their places
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const std::uint32_t t = 32 * ti + 8 * (r / 4) + 4 * hh + r % 4;
-    kl[t][col] = uk[r];
-    vl[t][col] = wv[r];
-    out[0 * kC * kD + t * kD + col] = uk[r];
-    out[2 * kC * kD + t * kD + col] = wv[r];
-  }
-  __syncthreads();
-  // Qe = diag(gamma) Q - P Uk and Ov = P Wv
-  V16F qe, ov = {};
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const std::uint32_t t = 32 * ti + 8 * (r / 4) + 4 * hh + r % 4;
-    qe[r] = Gm[t] * ql[t][col];
-  }
-#pragma unroll 2
-  for (int sb = 0; sb < 8; ++sb) {
-    const float4 pa = *reinterpret_cast<const float4*>(&pm[32 * ti + fr][4 * sb + 32 * hh]);
-    const float pv[4] = {pa.x, pa.y, pa.z, pa.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const std::uint32_t tok = 4 * sb + e + 32 * hh;
-      qe = __builtin_amdgcn_mfma_f32_32x32x2f32(-pv[e], kl[tok][col], qe, 0, 0, 0);
-      ov = __builtin_amdgcn_mfma_f32_32x32x2f32(pv[e], vl[tok][col], ov, 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const std::uint32_t t = 32 * ti + 8 * (r / 4) + 4 * hh + r % 4;
-    out[1 * kC * kD + t * kD + col] = qe[r];
-    out[3 * kC * kD + t * kD + col] = ov[r];
-  }
-  if (tid < kC) Gc[(static_cast<std::size_t>(c) * Hv + h) * kC + tid] = G[tid];
+  // the scan's weights: exp(G_C - G_t) of token t, 0 past the end; the last word, whose weight is 1 in a whole chunk and
+  // 0 in a shorter one, holds gamma_C instead
+  if (tid < kC)
+    Wt[(static_cast<std::size_t>(c) * Hv + h) * kC + tid] =
+        tid == kC - 1 ? Gm[kC - 1] : tid < L ? expf((G[kC - 1] - G[tid]) + (Gl[kC - 1] - Gl[tid])) : 0.0f;
 }
 
-// grid (n_seq * Hv * 128 / kNC), block 512 (8 waves): block -> (sequence, head, kNC value columns); walks
-// the sequence's chunks carrying its 128 x kNC slice of S in LDS. kNC = 32 (four blocks per head): each chunk's Uk,
-// Qe and K are read by four blocks (measured on C3: 16 columns per block 910 us, 32 878 us, 64 1339 us; narrower
-// slices re-read more, wider ones leave fewer waves per head for the chunk-serial MFMA work).
-// MFMA v_mfma_f32_16x16x4f32 (A lane l = A[l % 16][k], B lane l = B[k][l % 16], D lane l holds column l % 16 and
-// rows 4 (l / 16) + r) with each lane's k contiguous: lane quarter fq takes k in [K/4 fq, K/4 (fq + 1)), so every
-// operand read is 16 bytes (4 steps); a wave's four column tiles are four independent accumulator chains. The LDS
-// tiles that serve as B or as a transposed A are stored transposed: S as st[column][key], Delta as dt[column][token],
-// K as kt[key][token] (kt reuses Uk's space once Uk has been read).
-// Per chunk: waves 0-3 form Delta rows 16 w .. + 16 (= Wv - Uk S0), waves 4-7 the output rows (Qe S0 + Ov), four
-// 16-column tiles each; then wave w updates S rows 16 w .. + 16. The next chunk's operands are loaded into registers
-// during the current one; the block barriers inside the chunk loop synchronize LDS only, so those loads stay in
-// flight across them.
-// Column of token `tok` in row `key` of the K^T tile: 4-token groups xor-swizzled by (key / 8) & 15. With the 72-float
-// row stride, both the transposed 4-byte stores (64 lanes: 16 key rows x 4 tokens) and the 16-byte operand reads (16
-// key rows, one 4-token group) land on distinct banks of the 64-bank LDS.
-__device__ __forceinline__ std::uint32_t KtCol(std::uint32_t key, std::uint32_t tok) {
-  return 4 * ((tok / 4) ^ ((key / 8) & 15)) + tok % 4;
-}
-
+// grid (n_seq * Hv * 128 / kNC), block 512 (8 waves): block -> (sequence, kNC value columns, head); walks the sequence's
+// chunks carrying its 128 x kNC slice of S. MFMA v_mfma_f32_16x16x4f32 (A lane l = A[l % 16][k], B lane l = B[k][l % 16],
+// D lane l holds column l % 16 and rows 4 (l / 16) + r); instruction (sb, e) takes k = 16 sb + 4 (l / 16) + e, so every
+// operand is 16 bytes of a row for four instructions.
+// Per chunk: waves 0-3 form Delta rows 16 w .. + 16 (= Wv - Uk S0), waves 4-7 the output rows (Qe S0 + Ov); then wave w
+// updates S rows (keys) 16 w .. + 16, which it keeps in its accumulators for the whole sequence.
+// What bounds it: the chunk-serial path of one block (a long sequence has one block per CU), so everything off that path
+// is off it: Uk, Qe, K, Wv, Ov and the weights are read once by exactly the lanes that multiply them, so they come
+// from memory straight into operand registers, one chunk ahead (each register is reloaded as soon as its chunk has used
+// it); LDS holds only what the waves exchange, S^T and Delta^T, with two barriers per chunk. The loads stand among
+// the products: issued behind them, they take the vector memory pipe as long again as half the products. (Staging the
+// operands in LDS: 515 us for 8000 tokens in slices of 16 columns, 720 us for the ragged batch in slices of 32; this 440
+// and 590.)
+// h varies fastest over the grid: a head's slices land on one XCD (Hv % 8 == 0), whose L2 they share.
 template <typename In, int kNC>
 __device__ __forceinline__ void WyScan(const In* __restrict__ k, const float* __restrict__ wy,
-                                       const float* __restrict__ Gc, const std::uint32_t* __restrict__ chunks,
+                                       const float* __restrict__ Wt, const std::uint32_t* __restrict__ chunks,
                                        const std::uint32_t* __restrict__ seqs, float* __restrict__ state,
                                        float* __restrict__ o, std::uint32_t Hv, std::uint32_t Hk) {
-  constexpr int kNB = kD / kNC, kNT = kNC / 16, kTL = kC + 8, kDL = kC + 4, kStL = kD + 4, kWL = kNC + 4;
-  constexpr int kUkF = kC * kCL, kKtF = kD * kTL, kAF = kUkF > kKtF ? kUkF : kKtF;
-  __shared__ __attribute__((aligned(16))) float ua[kAF];       // Uk [64][kCL], then K^T [128][kTL]
-  __shared__ __attribute__((aligned(16))) float qel[kC][kCL];
+  constexpr int kNB = kD / kNC, kNT = kNC / 16, kDL = kC + 4, kStL = kD + 4;
   __shared__ __attribute__((aligned(16))) float st[kNC][kStL];  // S^T slice: [column][key]
   __shared__ __attribute__((aligned(16))) float dt[kNC][kDL];   // Delta^T slice: [column][token]
-  __shared__ __attribute__((aligned(16))) float wvl[kC][kWL];
-  __shared__ __attribute__((aligned(16))) float ovl[kC][kWL];
-  __shared__ __attribute__((aligned(16))) float Gl[kC], Wl[kC];
-  float(*ukl)[kCL] = reinterpret_cast<float(*)[kCL]>(ua);
-  float(*kt)[kTL] = reinterpret_cast<float(*)[kTL]>(ua);
-  // Blocks are dispatched in id order and a block's LDS leaves room for one per CU, so the longest sequences take
-  // the lowest ids (rank by descending chunk count, ties by index; up to 64 sequences, else in order): the chunk-
-  // serial critical path starts first.
+  // Blocks are dispatched in id order, so the longest sequences take the lowest ids (rank by descending chunk count, ties
+  // by index; up to 64 sequences, else in order): the chunk-serial critical path starts first.
   __shared__ std::uint32_t sq_s;
-  const std::uint32_t b = blockIdx.x, cb = b % kNB, h = (b / kNB) % Hv, rank = b / (kNB * Hv);
+  const std::uint32_t b = blockIdx.x, h = b % Hv, cb = (b / Hv) % kNB, rank = b / (kNB * Hv);
   const std::uint32_t n_seq = gridDim.x / (kNB * Hv);
   if (threadIdx.x == 0) {
     std::uint32_t pick = rank;
@@ -342,186 +403,166 @@ __device__ __forceinline__ void WyScan(const In* __restrict__ k, const float* __
     sq_s = pick;
   }
   __syncthreads();
-  const std::uint32_t sq = sq_s, kh = h % Hk;
-  const std::uint32_t tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, fc = lane % 16, fq = lane / 16;
-  const std::uint32_t j0 = cb * kNC;
+  const std::uint32_t sq = __builtin_amdgcn_readfirstlane(sq_s), kh = h % Hk;
+  const std::uint32_t tid = threadIdx.x, lane = tid % kWave, fc = lane % 16, fq = lane / 16;
+  const std::uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const std::uint32_t j0 = cb * kNC, r0 = 16 * (wave % 4), s0 = 16 * wave;
+  const bool delta = wave < 4;
   const std::uint32_t c0 = seqs[sq * 2], nc = seqs[sq * 2 + 1];
+  if (nc == 0) return;
   // a sequence's chunks are consecutive 64-token runs: chunk ci starts at first + 64 ci and holds
   // min(64, len - 64 ci) tokens (no chunk-table read per chunk: those scalar loads sat on the serial path)
-  const std::uint32_t first = nc ? chunks[c0 * 3] : 0u;
-  const std::uint32_t len = nc ? chunks[(c0 + nc - 1) * 3] + chunks[(c0 + nc - 1) * 3 + 1] - first : 0u;
+  const std::uint32_t first = chunks[c0 * 3];
+  const std::uint32_t len = chunks[(c0 + nc - 1) * 3] + chunks[(c0 + nc - 1) * 3 + 1] - first;
   float* Sg = state + (static_cast<std::size_t>(sq) * Hv + h) * kD * kD;
-  // S slice into st: 128 keys x kNC columns, kNC / 16 float4 per thread (key (tid / (kNC / 4)) + (2048 / kNC) i,
-  // columns 4 (tid % (kNC / 4)))
+  V4F S[kNT];  // S[s0 + 4 fq + i][j0 + 16 ct + fc]
 #pragma unroll
-  for (int i = 0; i < kNT; ++i) {
-    const std::uint32_t r = tid / (kNC / 4) + (2048 / kNC) * i, p = tid % (kNC / 4);
-    const float4 v4 = *reinterpret_cast<const float4*>(Sg + static_cast<std::size_t>(r) * kD + j0 + 4 * p);
-    st[4 * p][r] = v4.x, st[4 * p + 1][r] = v4.y, st[4 * p + 2][r] = v4.z, st[4 * p + 3][r] = v4.w;
+  for (int ct = 0; ct < kNT; ++ct) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[ct][i] = Sg[static_cast<std::size_t>(s0 + 4 * fq + i) * kD + j0 + 16 * ct + fc];
+    *reinterpret_cast<float4*>(&st[16 * ct + fc][s0 + 4 * fq]) = make_float4(S[ct][0], S[ct][1], S[ct][2], S[ct][3]);
   }
-  // staged operands of one chunk, in registers: Uk, Qe (8192 floats each: 4 float4 per thread), the Wv and Ov slices
-  // (64 x 64 each: rows tid / 16 and tid / 16 + 32, columns 4 (tid % 16)), G (threads < 64); K (8192 inputs: two
-  // packs of 8) on its own, since it is stored later in the chunk
-  // Wv / Ov slices: 64 x kNC floats = 16 kNC float4, float4 e = tid + 512 i at row e / (kNC / 4), column 4 (e % (kNC / 4));
-  // with kNC = 16 the first 256 threads hold one each
-  constexpr int kWN = (kC * kNC / 4 + 511) / 512;
-  constexpr bool kWAll = kC * kNC / 4 >= 512;
-  float4 ru0, ru1, ru2, ru3, rq0, rq1, rq2, rq3, rw[kWN], ro[kWN];
-  Pack8<In> rk0, rk1;
-  float rg;
-  auto load = [&](std::uint32_t ci) {
-    const std::uint32_t c = c0 + ci;
-    const float* base = wy + (static_cast<std::size_t>(c) * Hv + h) * 4 * kC * kD;
-    const float4* bu = reinterpret_cast<const float4*>(base);
-    const float4* bq = reinterpret_cast<const float4*>(base + kC * kD);
-    ru0 = bu[tid], ru1 = bu[tid + 512], ru2 = bu[tid + 1024], ru3 = bu[tid + 1536];
-    rq0 = bq[tid], rq1 = bq[tid + 512], rq2 = bq[tid + 1024], rq3 = bq[tid + 1536];
-    const std::uint32_t t = tid / (kNC / 4), p = 4 * (tid % (kNC / 4));
-    const float* bw = base + 2 * kC * kD + j0 + p;
-    const float* bo = base + 3 * kC * kD + j0 + p;
+  // this lane's operands of the chunk to come: A rows of Uk or Qe, the Wv or Ov values its results join, K^T rows, weights
+  float4 ra[8], rw[4];
+  float rv[kNT][4], rk[16];
+  const std::size_t tile = kC * kD, step = static_cast<std::size_t>(Hv) * 4 * tile;
+  const float* pa = wy + (static_cast<std::size_t>(c0) * Hv + h) * 4 * tile;  // Uk, Qe, Wv, Ov of the chunk to load
+  const float* pw = Wt + (static_cast<std::size_t>(c0) * Hv + h) * kC;
+  const std::uint32_t aoff = (delta ? 0u : kC * kD) + (r0 + fc) * kD + 4 * fq;
+  const std::uint32_t voff = (delta ? 2u : 3u) * kC * kD + (r0 + 4 * fq) * kD + j0 + fc;
+  const auto load_a = [&](int sb) { ra[sb] = *reinterpret_cast<const float4*>(pa + aoff + 16 * sb); };
+  const auto load_v = [&]() {
 #pragma unroll
-    for (int i = 0; i < kWN; ++i)
-      if (kWAll || tid < kC * kNC / 4) {
-        rw[i] = *reinterpret_cast<const float4*>(bw + (t + (2048 / kNC) * i) * kD);
-        ro[i] = *reinterpret_cast<const float4*>(bo + (t + (2048 / kNC) * i) * kD);
-      }
-    rg = Gc[(static_cast<std::size_t>(c) * Hv + h) * kC + tid % kC];
+    for (int ct = 0; ct < kNT; ++ct)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rv[ct][i] = pa[voff + i * kD + 16 * ct];
   };
-  auto load_k = [&](std::uint32_t ci) {
+  // K^T row s0 + fc, tokens 16 sb + 4 fq + e: a uniform row address plus the lane's offset; rows past a short chunk's end
+  // reload its last one (their weights are zero)
+  const std::uint32_t kstride = Hk * kD;
+  const auto load_k = [&](std::uint32_t ci, int sb) {
     const std::uint32_t start = first + 64 * ci, L = min(64u, len - 64 * ci);
-    const std::uint32_t t0 = tid / 16, p8 = 8 * (tid % 16);  // packs tid and tid + 512: rows t0 and t0 + 32
-    rk0 = Ld8(k + (static_cast<std::size_t>(start + min(t0, L - 1)) * Hk + kh) * kD + p8);
-    rk1 = Ld8(k + (static_cast<std::size_t>(start + min(t0 + 32, L - 1)) * Hk + kh) * kD + p8);
-  };
-  auto store = [&]() {
-    // float4 e = tid + 512 i of a 64 x 128 tile is row e / 32 = tid / 32 + 16 i, column 4 (tid % 32)
-    const std::uint32_t t0 = tid / 32, p4 = 4 * (tid % 32);
-    *reinterpret_cast<float4*>(&ukl[t0][p4]) = ru0;
-    *reinterpret_cast<float4*>(&ukl[t0 + 16][p4]) = ru1;
-    *reinterpret_cast<float4*>(&ukl[t0 + 32][p4]) = ru2;
-    *reinterpret_cast<float4*>(&ukl[t0 + 48][p4]) = ru3;
-    *reinterpret_cast<float4*>(&qel[t0][p4]) = rq0;
-    *reinterpret_cast<float4*>(&qel[t0 + 16][p4]) = rq1;
-    *reinterpret_cast<float4*>(&qel[t0 + 32][p4]) = rq2;
-    *reinterpret_cast<float4*>(&qel[t0 + 48][p4]) = rq3;
-    const std::uint32_t t = tid / (kNC / 4), p = 4 * (tid % (kNC / 4));
+    const In* kc = k + (static_cast<std::size_t>(start) * Hk + kh) * kD;
 #pragma unroll
-    for (int i = 0; i < kWN; ++i)
-      if (kWAll || tid < kC * kNC / 4) {
-        *reinterpret_cast<float4*>(&wvl[t + (2048 / kNC) * i][p]) = rw[i];
-        *reinterpret_cast<float4*>(&ovl[t + (2048 / kNC) * i][p]) = ro[i];
-      }
-    if (tid < kC) Gl[tid] = rg;
+    for (int e = 0; e < 4; ++e) rk[4 * sb + e] = Cv(kc[__umul24(min(16u * sb + 4 * fq + e, L - 1), kstride) + s0 + fc]);
+    rw[sb] = *reinterpret_cast<const float4*>(pw + 16 * sb + 4 * fq);
   };
-  auto store_k = [&](std::uint32_t L) {
-    const std::uint32_t tk = tid / 16, pk = 8 * (tid % 16);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      kt[pk + e][KtCol(pk + e, tk)] = tk < L ? Cv(rk0.v[e]) : 0.0f;
-      kt[pk + e][KtCol(pk + e, tk + 32)] = tk + 32 < L ? Cv(rk1.v[e]) : 0.0f;
-    }
-  };
+  for (int sb = 0; sb < 8; ++sb) load_a(sb);
+  load_v();
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) load_k(0, sb);
+  float gc = pw[kC - 1];
   const float inv_sqrt_d = 1.0f / sqrtf(static_cast<float>(kD));
-  if (nc > 0) {
-    load(0);
-    load_k(0);
-  }
+  halo::LdsSync();
   for (std::uint32_t ci = 0; ci < nc; ++ci) {
     const std::uint32_t start = first + 64 * ci, L = min(64u, len - 64 * ci), cn = ci + 1 < nc ? ci + 1 : ci;
-    store();
-    halo::LdsSync();
-    load(cn);  // unconditional (the last chunk reloads itself): no loads under a branch
-    if (tid < kC) Wl[tid] = expf(Gl[kC - 1] - Gl[tid]);  // the S-update weights exp(G_C - G_t)
-    // Delta (waves 0-3) or the output (waves 4-7): token rows 16 (w % 4) .. + 16, four 16-column tiles, K range =
-    // 128 keys, lane keys 32 fq .. + 32
-    {
-      const std::uint32_t r0 = 16 * (wave % 4);
-      float(*A)[kCL] = wave < 4 ? ukl : qel;
-      V4F acc[kNT];
+    if (cn != ci) pa += step, pw += static_cast<std::size_t>(Hv) * kC;  // the last chunk reloads itself
+    V4F acc[kNT][2];
 #pragma unroll
-      for (int ct = 0; ct < kNT; ++ct) acc[ct] = V4F{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 2
-      for (int sb = 0; sb < 8; ++sb) {
-        const float4 av = *reinterpret_cast<const float4*>(&A[r0 + fc][32 * fq + 4 * sb]);
+    for (int ct = 0; ct < kNT; ++ct) acc[ct][0] = acc[ct][1] = V4F{0.0f, 0.0f, 0.0f, 0.0f};
+    // operand rows of S^T in groups of kG steps, each read ahead of the group before it
+    constexpr int kG = 2;
+    float4 bv[2][kG][kNT];
+    const auto read_s = [&](int g) {
+#pragma unroll
+      for (int i = 0; i < kG; ++i)
+#pragma unroll
+        for (int ct = 0; ct < kNT; ++ct)
+          bv[g % 2][i][ct] = *reinterpret_cast<const float4*>(&st[16 * ct + fc][16 * (kG * g + i) + 4 * fq]);
+    };
+    read_s(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < 8 / kG; ++g) {
+      if (g + 1 < 8 / kG) read_s(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const int sb = kG * g + i;
+        const float4 av = ra[sb];
 #pragma unroll
         for (int ct = 0; ct < kNT; ++ct) {
-          const float4 bv = *reinterpret_cast<const float4*>(&st[16 * ct + fc][32 * fq + 4 * sb]);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, bv.x, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, bv.y, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, bv.z, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, bv.w, acc[ct], 0, 0, 0);
+          const float4 x = bv[g % 2][i][ct];
+          V4F& a = acc[ct][sb % 2];  // two chains
+          a = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, x.x, a, 0, 0, 0);
+          a = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, x.y, a, 0, 0, 0);
+          a = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, x.z, a, 0, 0, 0);
+          a = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, x.w, a, 0, 0, 0);
         }
+        load_a(sb);  // among the products: issued together after them, the loads took as long as half the products
+        __builtin_amdgcn_sched_barrier(0);
       }
+    }
 #pragma unroll
-      for (int ct = 0; ct < kNT; ++ct) {
-        const std::uint32_t col = 16 * ct + fc;
-        if (wave < 4) {
-          float d4[4];
+    for (int ct = 0; ct < kNT; ++ct) {
+      const V4F a = acc[ct][0] + acc[ct][1];
+      if (delta) {
+        *reinterpret_cast<float4*>(&dt[16 * ct + fc][r0 + 4 * fq]) =
+            make_float4(rv[ct][0] - a[0], rv[ct][1] - a[1], rv[ct][2] - a[2], rv[ct][3] - a[3]);
+      } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) d4[i] = wvl[r0 + 4 * fq + i][col] - acc[ct][i];
-          *reinterpret_cast<float4*>(&dt[col][r0 + 4 * fq]) = make_float4(d4[0], d4[1], d4[2], d4[3]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const std::uint32_t t = r0 + 4 * fq + i;
-            if (t < L)
-              o[(static_cast<std::size_t>(start + t) * Hv + h) * kD + j0 + col] = (acc[ct][i] + ovl[t][col]) * inv_sqrt_d;
-          }
+        for (int i = 0; i < 4; ++i) {
+          const std::uint32_t t = r0 + 4 * fq + i;
+          if (t < L) o[(static_cast<std::size_t>(start + t) * Hv + h) * kD + j0 + 16 * ct + fc] = (a[i] + rv[ct][i]) * inv_sqrt_d;
         }
       }
     }
-    halo::LdsSync();
-    store_k(L);  // Uk has been read: K^T takes its place
-    load_k(cn);
-    halo::LdsSync();
-    // S rows 16 w .. + 16, four 16-column tiles: gamma_C S + (K diag(exp(G_C - G_t)))^T Delta, K range = 64 tokens,
-    // lane tokens 16 fq .. + 16
-    {
-      const std::uint32_t r0 = 16 * wave;
-      const float gc = expf(Gl[kC - 1]);
-      V4F acc[kNT];
+    load_v();
+    halo::LdsSync();  // Delta^T is whole, S^T has been read
+    // S rows: gamma_C S + (K diag(W))^T Delta over 64 tokens
+    V4F upd[kNT];
+#pragma unroll
+    for (int ct = 0; ct < kNT; ++ct) S[ct] *= gc, upd[ct] = V4F{0.0f, 0.0f, 0.0f, 0.0f};
+    gc = pw[kC - 1];
+    float4 dv[4][kNT];
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb)
+#pragma unroll
+      for (int ct = 0; ct < kNT; ++ct) dv[sb][ct] = *reinterpret_cast<const float4*>(&dt[16 * ct + fc][16 * sb + 4 * fq]);
+    float ka[16];  // K^T diag(W): while Delta^T arrives
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb) {
+      ka[4 * sb] = rk[4 * sb] * rw[sb].x, ka[4 * sb + 1] = rk[4 * sb + 1] * rw[sb].y;
+      ka[4 * sb + 2] = rk[4 * sb + 2] * rw[sb].z;
+      ka[4 * sb + 3] = rk[4 * sb + 3] * (sb == 3 && fq == 3 ? (L == 64 ? 1.0f : 0.0f) : rw[sb].w);  // W[63]: gamma_C
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb) {
+      load_k(cn, sb);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ct = 0; ct < kNT; ++ct) {
-        const float4 s4 = *reinterpret_cast<const float4*>(&st[16 * ct + fc][r0 + 4 * fq]);
-        acc[ct][0] = gc * s4.x, acc[ct][1] = gc * s4.y, acc[ct][2] = gc * s4.z, acc[ct][3] = gc * s4.w;
+        V4F& u = sb % 2 ? upd[ct] : S[ct];
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[4 * sb], dv[sb][ct].x, u, 0, 0, 0);
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[4 * sb + 1], dv[sb][ct].y, u, 0, 0, 0);
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[4 * sb + 2], dv[sb][ct].z, u, 0, 0, 0);
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[4 * sb + 3], dv[sb][ct].w, u, 0, 0, 0);
       }
+    }
 #pragma unroll
-      for (int sb = 0; sb < 4; ++sb) {
-        const std::uint32_t tk = 16 * fq + 4 * sb;
-        const float4 kv = *reinterpret_cast<const float4*>(&kt[r0 + fc][KtCol(r0 + fc, tk)]);
-        const float4 wv = *reinterpret_cast<const float4*>(&Wl[tk]);
-        const float a0 = kv.x * wv.x, a1 = kv.y * wv.y, a2 = kv.z * wv.z, a3 = kv.w * wv.w;
-#pragma unroll
-        for (int ct = 0; ct < kNT; ++ct) {
-          const float4 dv = *reinterpret_cast<const float4*>(&dt[16 * ct + fc][tk]);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, dv.x, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, dv.y, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, dv.z, acc[ct], 0, 0, 0);
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a3, dv.w, acc[ct], 0, 0, 0);
-        }
-      }
-#pragma unroll
-      for (int ct = 0; ct < kNT; ++ct)
-        *reinterpret_cast<float4*>(&st[16 * ct + fc][r0 + 4 * fq]) = make_float4(acc[ct][0], acc[ct][1], acc[ct][2], acc[ct][3]);
+    for (int ct = 0; ct < kNT; ++ct) {
+      S[ct] += upd[ct];
+      *reinterpret_cast<float4*>(&st[16 * ct + fc][s0 + 4 * fq]) = make_float4(S[ct][0], S[ct][1], S[ct][2], S[ct][3]);
     }
     halo::LdsSync();
   }
 #pragma unroll
-  for (int i = 0; i < kNT; ++i) {
-    const std::uint32_t r = tid / (kNC / 4) + (2048 / kNC) * i, p = tid % (kNC / 4);
-    *reinterpret_cast<float4*>(Sg + static_cast<std::size_t>(r) * kD + j0 + 4 * p) =
-        make_float4(st[4 * p][r], st[4 * p + 1][r], st[4 * p + 2][r], st[4 * p + 3][r]);
-  }
+  for (int ct = 0; ct < kNT; ++ct)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) Sg[static_cast<std::size_t>(s0 + 4 * fq + i) * kD + j0 + 16 * ct + fc] = S[ct][i];
 }
+}  // namespace
 
-extern "C" __global__ void __launch_bounds__(512)
+extern "C" __global__ void __launch_bounds__(512, 4)
     halo_gdn_wy_prep(const std::uint16_t* __restrict__ q, const std::uint16_t* __restrict__ k,
                      const std::uint16_t* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta,
                      const std::uint32_t* __restrict__ chunks, float* __restrict__ wy, float* __restrict__ Gc,
                      std::uint32_t Hv, std::uint32_t Hk) {
   WyPrep(q, k, v, g, beta, chunks, wy, Gc, Hv, Hk);
 }
-extern "C" __global__ void __launch_bounds__(512)
+extern "C" __global__ void __launch_bounds__(512, 4)
     halo_gdn_wy_prep_f32(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
                          const float* __restrict__ g, const float* __restrict__ beta,
                          const std::uint32_t* __restrict__ chunks, float* __restrict__ wy, float* __restrict__ Gc,

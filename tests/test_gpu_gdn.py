@@ -230,3 +230,13 @@ def test_gdn_prefill_single_sequence_slices(dev):
                                                      g[:n], beta[:n]), range(32))
     _close(one_o, want_o, "outputs")
     _close(one_s, want_s, "final state")
+
+
+@pytest.mark.parametrize("seqlens", [[1], [16, 17], [63, 64, 65], [48, 129, 2]])
+def test_gdn_prefill_tile_edges(dev, seqlens):
+    """Sequence lengths at the edges of the 16-token tiles and 64-token chunks: every head against stepping, within 1e-5 of
+    each value's term magnitude (the bound of the C3 test)."""
+    go, gs, state0, inputs = prefill_case(dev, np.random.default_rng(sum(seqlens)), seqlens)
+    wo, ws_, mo, ms = oracle_prefill_all(seqlens, state0, inputs)
+    _close_mag(go, wo, mo, "outputs")
+    _close_mag(gs, ws_, ms, "final state")
