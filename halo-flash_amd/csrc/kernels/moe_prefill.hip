@@ -148,12 +148,15 @@ extern "C" __global__ void __launch_bounds__(1024)
   __syncthreads();
   if (g <= E) {
     start[g] = c[g];
-    const std::uint32_t first = tcount[g];
-    for (std::uint32_t i = 0; i * tile < n; ++i) {
+    const std::uint32_t first = tcount[g], nt = (n + tile - 1) / tile;
+    // the group's tiles in like sizes of whole 32s (the waves of a tile work in 32s: 156 pairs as 96 + 60, not 128 + 28)
+    const std::uint32_t each = nt ? ((n + nt - 1) / nt + 31) / 32 * 32 : 0;
+    for (std::uint32_t i = 0; i < nt; ++i) {
       std::uint32_t* tt = tiles + 3 * static_cast<std::size_t>(first + i);
+      const std::uint32_t at = min(i * each, n);
       tt[0] = g;
-      tt[1] = c[g] + i * tile;
-      tt[2] = min(tile, n - i * tile);
+      tt[1] = c[g] + at;
+      tt[2] = min(each, n - at);
     }
   }
 }

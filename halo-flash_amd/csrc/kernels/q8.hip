@@ -913,7 +913,12 @@ __device__ __forceinline__ void GemmTileQ8(const std::int8_t* __restrict__ A0, c
 // Tile rows are 64 bytes with the 16-byte chunk index xor-swizzled by (row >> 2) & 3, which keeps the fragment reads
 // (32 consecutive rows, one chunk each) free of bank conflicts. The stage loop is unrolled by three so every LDS
 // address is a per-lane constant plus an immediate. The scale MFMA is the two-block rank-1 v_mfma_f32_32x32x1_2b,
-// covering two tiles (NMAT * MT even) or both blocks of the stage (a single tile).
+// covering two tiles (NMAT * MT even) or both blocks of the stage (a single tile). The activations are the A operand, so
+// that a result register holds one token's values of 32 consecutive matrix rows across its lanes.
+// What bounds it: issue slots. Each 32 x 32 tile and block takes 32 convert / FMA instructions beside its matrix
+// instructions; both together fill 72% of the issue slots at two blocks per CU. (Measured and not kept: products of
+// the next block issued before the current one's additions, 172 VGPRs and one block per CU: 10% slower.) 8192 x 2048 at
+// 8000 tokens: 416 -> 404 us with the activations as A operand (stores of 128 bytes instead of 32).
 // Limits: cols % 64 == 0; every weight offset (rows * qstride) and activation offset fits in 32 bits.
 using halo::DmaDword;
 using halo::DmaRow16;
@@ -947,7 +952,11 @@ __device__ __forceinline__ void GemmTileQ8Dma(const std::int8_t* __restrict__ A0
   __shared__ __attribute__((aligned(1024))) std::int8_t lds[3 * STAGE];
   const std::uint32_t tid = threadIdx.x, lane = tid % 64;
   const std::uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const std::uint32_t wr = wave / WT, wt = wave % WT;
+  // A wave whose 32 tokens lie past the tile's end stages and waits with the others but multiplies nothing; which wave of
+  // a row (and so which SIMD: waves go round the four) that is differs from block to block, so a CU's blocks idle
+  // different SIMDs.
+  const std::uint32_t wr = wave / WT, wt = (wave + blockIdx.x + blockIdx.y) % WT;
+  const bool live = wt * 32 < ntok;
   const std::uint32_t nblk = cols / 32, nk = cols / 64;
   const std::uint32_t lbase = static_cast<std::uint32_t>(reinterpret_cast<std::uintptr_t>(lds));
   const auto tokrow = [&](std::uint32_t i) {
@@ -1021,12 +1030,12 @@ __device__ __forceinline__ void GemmTileQ8Dma(const std::int8_t* __restrict__ A0
     if constexpr (NT == 1) {
       const float dw = F16(*reinterpret_cast<const std::uint16_t*>(sb + dwo));
       const float sx = *reinterpret_cast<const float*>(sb + sxo);
-      const V32F32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, sx, fz, 0, 0, 0);
+      const V32F32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(sx, dw, fz, 0, 0, 0);
       const V4i af0 = *reinterpret_cast<const V4i*>(sb + a0), af1 = *reinterpret_cast<const V4i*>(sb + (a0 ^ 32u));
       const V4i bf0 = *reinterpret_cast<const V4i*>(sb + RB + b0);
       const V4i bf1 = *reinterpret_cast<const V4i*>(sb + RB + (b0 ^ 32u));
-      const V16I32 c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(af0, bf0, z, 0, 0, 0);
-      const V16I32 c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(af1, bf1, z, 0, 0, 0);
+      const V16I32 c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf0, af0, z, 0, 0, 0);
+      const V16I32 c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf1, af1, z, 0, 0, 0);
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[0][j] = __builtin_fmaf(static_cast<float>(c0[j]), sc[j], acc[0][j]);
 #pragma unroll
@@ -1046,11 +1055,11 @@ __device__ __forceinline__ void GemmTileQ8Dma(const std::int8_t* __restrict__ A0
             __builtin_amdgcn_s_setprio(PRIO);  // issue this wave's MFMAs ahead of other waves' epilogues
           }
           const float dw = F16(*reinterpret_cast<const std::uint16_t*>(sb + dwo + tile_row_off(p0) + blk * 2));
-          const V32F32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, sx, fz, 0, 0, 0);
+          const V32F32 sc = __builtin_amdgcn_mfma_f32_32x32x1f32(sx, dw, fz, 0, 0, 0);
           const V4i af0 = *reinterpret_cast<const V4i*>(sb + ao + (p0 / MT) * ROWS * 64 + (p0 % MT) * 2048);
           const V4i af1 = *reinterpret_cast<const V4i*>(sb + ao + (p1 / MT) * ROWS * 64 + (p1 % MT) * 2048);
-          const V16I32 c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(af0, bf, z, 0, 0, 0);
-          const V16I32 c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(af1, bf, z, 0, 0, 0);
+          const V16I32 c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af0, z, 0, 0, 0);
+          const V16I32 c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af1, z, 0, 0, 0);
           if constexpr (PRIO) {
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_setprio(0);
@@ -1073,9 +1082,11 @@ __device__ __forceinline__ void GemmTileQ8Dma(const std::int8_t* __restrict__ A0
     WaitVmem<SPR + SPS>();
     __builtin_amdgcn_s_barrier();
     issue(min(kc + 2, nk - 1), (B + 2) % 3);
-    compute(bufc);
+    if (live) {
+      compute(bufc);
 #pragma unroll
-    for (int p = 0; p < NT; ++p) PinVgprs(acc[p]);  // the stage's epilogue stays in the stage
+      for (int p = 0; p < NT; ++p) PinVgprs(acc[p]);  // the stage's epilogue stays in the stage
+    }
   };
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
@@ -1091,25 +1102,19 @@ __device__ __forceinline__ void GemmTileQ8Dma(const std::int8_t* __restrict__ A0
   if (kc < nk) stage(kc++, B0{});
   if (kc < nk) stage(kc++, B1{});
   WaitVmem<0>();  // no DMA may land after the block's LDS is released
-  if (tok >= ntok) return;
-  float* yt = y + static_cast<std::size_t>(yrow0 + tok) * ystride;
+  // lane l holds matrix row l % 32 of each tile and tokens 8 (j / 4) + 4 (l / 32) + j % 4: 32 lanes store 128 consecutive
+  // bytes of a token's row (with tokens across the lanes the same stores were 32-byte pieces of 32 rows)
+  if (!live) return;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int mt = 0; mt < MT; ++mt) {
+    const std::uint32_t r = r0 + wr * MT * 32 + mt * 32 + fr;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const std::uint32_t r = r0 + wr * MT * 32 + mt * 32 + g * 8 + fh * 4;
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] = NMAT == 2 ? Silu(acc[mt][4 * g + e]) * acc[MT + mt][4 * g + e] : acc[mt][4 * g + e];
-      if (r + 3 < rows && ystride % 4 == 0) {
-        *reinterpret_cast<float4*>(yt + r) = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (r + e < rows) yt[r + e] = v[e];
-      }
+    for (int j = 0; j < 16; ++j) {
+      const std::uint32_t t = wt * 32 + 8 * (j / 4) + 4 * fh + j % 4;
+      const float v = NMAT == 2 ? Silu(acc[mt][j]) * acc[MT + mt][j] : acc[mt][j];
+      if (t < ntok && r < rows) y[static_cast<std::size_t>(yrow0 + t) * ystride + r] = v;
     }
+  }
 }
 }  // namespace halo
 

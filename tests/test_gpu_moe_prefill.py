@@ -106,3 +106,10 @@ def test_moe_prefill_matches_oracle(dev, c2, small, shape, T):
         dec = outd.download()
         scale = np.abs(dec).max()
         assert np.all(np.abs(got - dec) <= 1e-3 * scale), "prefill and decode paths disagree"
+
+
+@pytest.mark.parametrize("T", [260, 560])
+def test_moe_prefill_split_groups(dev, c2, small, T):
+    """Groups a little over one tile (about 65 pairs in 64-pair tiles, 140 in 128-pair ones, the shared expert's group
+    several tiles): cut into like tiles of whole 32s, with waves past a tile's end idle."""
+    test_moe_prefill_matches_oracle(dev, c2, small, "small", T)
