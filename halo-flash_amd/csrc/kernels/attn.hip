@@ -1071,12 +1071,13 @@ __device__ __forceinline__ void AttnPrefill(
     }
     if (oq != nullptr) {  // a Q8 block is this step's 32 dims: 16 in each lane of the pair
       const float qs = fmaxf(amax, __shfl_xor(amax, 32)) / 127.0f;
+      const halo::CodeScale cs(qs);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         std::uint32_t word = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int code = qs > 0.0f ? static_cast<int>(rintf(v[4 * g + e] / qs)) : 0;
+          const int code = cs.Code(v[4 * g + e]);
           word |= (static_cast<std::uint32_t>(code) & 0xFFu) << (8 * e);
         }
         if (live) *reinterpret_cast<std::uint32_t*>(oq + qbase + d0 + 32 * c + 8 * g + 4 * h) = word;
