@@ -159,15 +159,30 @@ __device__ __forceinline__ void AttnDecodePartial(
   // queries of this kv head: slot i = session * G + g (prefix) or g (suffix)
   __shared__ __attribute__((aligned(16))) float knew[kFused ? 2 : 1][kFused ? kHd : 4];
   if constexpr (kFused) {
-    // wave w prepares queries w, w + 4, ... (the angles once per position)
+    // wave w prepares queries w, w + 4, ... (the angles once per position). The precise powf / cosf / sinf of a position cost
+    // more than the norms: two to four sessions' angles are formed by one wave each and shared through LDS (the scores'
+    // space): 4 sessions at 8576 positions 31.5 -> 30.8 us per layer.
     std::uint32_t cur = 0xFFFFFFFFu;
     halo::RopeCS cs{};
     float out[4];
+    float4* shared_cs = reinterpret_cast<float4*>(&sc[0][0]);
+    const bool share = kMma && is_prefix && S > 1 && S <= 4;
+    static_assert(sizeof(sc) >= 4 * kWave * sizeof(float4));
+    if (share) {
+      if (wave < S) {
+        cs = halo::RopeAngles(nkv[wave] - 1, rot, theta);
+        shared_cs[wave * kWave + lane] = make_float4(cs.c[0], cs.c[1], cs.s[0], cs.s[1]);
+      }
+      halo::LdsSync();
+    }
 #pragma unroll
     for (int m = 0; m < kQW; ++m) {
       const std::uint32_t qi = wave + 4u * m;
       if (qi >= nq) break;
-      if (qpos[m] != cur) {
+      if (share) {
+        const float4 v = shared_cs[qi / G * kWave + lane];
+        cs.c[0] = v.x, cs.c[1] = v.y, cs.s[0] = v.z, cs.s[1] = v.w;
+      } else if (qpos[m] != cur) {
         cur = qpos[m];
         cs = halo::RopeAngles(cur, rot, theta);
       }

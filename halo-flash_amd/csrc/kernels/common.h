@@ -451,6 +451,12 @@ __device__ __forceinline__ void NormRopeHead(const float (&x)[4], const float (&
 #pragma unroll
   for (int i = 0; i < 4; ++i) y[i] = x[i] * sc * w[i];
   const std::uint32_t half = rot / 2;
+  if (rot == 64) {  // every pair is (lane, lane ^ 32) of the first 64 dims: one exchange
+    const float partner = __shfl_xor(y[0], 32, kWave);
+    out[0] = lane < 32 ? y[0] * cs.c[0] - partner * cs.s[0] : partner * cs.s[0] + y[0] * cs.c[0];
+    out[1] = y[1], out[2] = y[2], out[3] = y[3];
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     out[i] = y[i];

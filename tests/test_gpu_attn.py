@@ -199,3 +199,27 @@ def test_attn_decode_step_equals_prep_then_decode(dev, S, prefix, suffixes, max_
     for s in range(S):
         row = outs[1][4][pages[s, last[s] // PAGE], :, last[s] % PAGE]
         assert np.array_equal(row, vin.download()[s])
+
+
+@pytest.mark.parametrize("S,rot", [(3, 32), (3, 128), (2, 64)])
+def test_attn_decode_step_shared_angles(dev, S, rot):
+    """Sessions at different positions behind a shared prefix: the blocks share each session's rotation angles between
+    their waves. Outputs and appended K bitwise those of halo_attn_prep_decode (angles per head) and
+    halo_op_attn_decode_q8, at rotary widths that pair dims within and across the first 64."""
+    rng = np.random.default_rng(rot + S)
+    Hkv, Hq, theta, eps, prefix, suffixes = 2, 16, 1e7, 1e-6, 128, [40, 3, 17][:S]
+    desc, g, kp, vp, pages, nkv = build(dev, rng, S, Hkv, prefix, suffixes, prefix + 64)
+    qg = dev.to_device(rng.normal(0, 1, (S, Hq, 2 * D)).astype(np.float32))
+    kin, vin = (dev.to_device(rng.normal(0, 1, (S, Hkv, D)).astype(np.float32)) for _ in range(2))
+    wq, wk = (dev.to_device(rng.normal(1, 0.1, D).astype(np.float32)) for _ in range(2))
+    ws = dev.array(H.lib().halo_op_attn_decode_workspace_bytes(ctypes.byref(desc), Hq), np.uint8)
+    o, q, gate = (dev.array((S, Hq, D), np.float32) for _ in range(3))
+    dev.op("attn_decode_step_q8", ctypes.byref(desc), qg.ptr, kin.ptr, vin.ptr, wq.ptr, wk.ptr, rot, theta, eps, o.ptr,
+           None, None, Hq, ws.ptr, ws.nbytes)
+    step, kpool = o.download(), g["k"].download()
+    dev.launch("halo_attn_prep_decode", (S, Hq + 2 * Hkv), (64,),
+               [qg, kin, vin, wq, wk, q, gate, g["k"], g["v"], g["pages"], g["nkv"], ("u32", Hq), ("u32", Hkv),
+                ("u32", desc.max_pages), ("u32", rot), ("f32", theta), ("f32", eps), None, None])
+    dev.op("attn_decode_q8", ctypes.byref(desc), q.ptr, gate.ptr, o.ptr, None, None, Hq, ws.ptr, ws.nbytes)
+    assert np.array_equal(step.view(np.uint32), o.download().view(np.uint32))
+    assert np.array_equal(kpool.view(np.uint32), g["k"].download().view(np.uint32))
