@@ -722,12 +722,12 @@ extern "C" __global__ void __launch_bounds__(64)
 // the conversions per query. One wave per SIMD hides nothing by itself, hence the hand-placed slices of vector work after each
 // matrix instruction. Registers: accumulators and most of Q in AGPRs (pinned; otherwise the compiler moves all 128
 // accumulators through VGPRs each chunk), no scratch.
-// One 8192-token prompt, 16 heads (550 GFLOP of fp32 products): 3.70 -> 1.67 ms = 329 TFLOP/s (988 of fp16 MFMA issue; a
+// One 8192-token prompt, 16 heads (550 GFLOP of fp32 products): 3.70 -> 1.70 ms = 323 TFLOP/s (970 of fp16 MFMA issue; a
 // large library bf16 matrix product reaches 1380 on this card). The form before held 16 queries per wave, 8 tokens per
 // block, with P through LDS.
 // AttnPrefill<2> (halo_attn_prefill_d2): 8-token tiles, two waves share 32 queries and split the output dims: 0.75x the
 // matrix work per wave and twice the blocks, for batches whose 8-token tiles fit the 256 CUs once (256 tokens at position
-// 8192: 840 us with 16-token tiles, 734 with these, measured on one build; 1167 before).
+// 8192: 840 us with 16-token tiles, 734 with these, on one build of this kernel; now 581, 1167 before).
 namespace {
 constexpr int kHalf = kChunk * kHd * 2;          // bytes of one staged matrix's hi (or lo) halves
 constexpr int kBuf = 2 * kHalf;                  // bytes of one staged chunk of K or V
