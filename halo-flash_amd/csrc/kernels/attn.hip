@@ -948,11 +948,12 @@ __device__ __forceinline__ void AttnPrefill(
     } else {
       ps = kSppT * (sva / kSvv);
     }
-    // the running max (base-2 units) lags by up to kLazy, so few chunks rescale
-    if (__any(cm > m + kLazy) || vfac != 1.0f) {
-      const float mx = fmaxf(m, cm);
-      const float alpha = mx == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mx);
-      m = mx;
+    // the running max (base-2 units) lags by up to kLazy, so few chunks rescale; a query's own scores decide when its max
+    // moves, so its bits do not depend on the queries that share its wave
+    const bool up = cm > m + kLazy;
+    if (__any(up) || vfac != 1.0f) {
+      const float alpha = up ? __builtin_amdgcn_exp2f(m - cm) : 1.0f;
+      m = up ? cm : m;
       l *= alpha;
 #pragma unroll
       for (int c = 0; c < NJ / 2; ++c) {

@@ -130,3 +130,50 @@ def test_attn_prefill_tile_shapes_bitwise(dev):
             pr /= pr.sum()
             sg = 1 / (1 + np.exp(-gate[p, h].astype(np.float64)))
             assert np.all(np.abs(whole[p, h] - pr @ V * sg) <= 1e-5 * (pr @ np.abs(V)) * sg + 1e-7), f"token {p} head {h}"
+
+
+def reference(q, gate, kp, vp, pages_s, p, h):
+    """One query's output in 64 bits and the magnitude of its terms, sum |p| |v| times the gate."""
+    K = gather(kp, pages_s, p + 1, h // 8).astype(np.float64)
+    V = gather(vp, pages_s, p + 1, h // 8).astype(np.float64)
+    sc = K @ q.astype(np.float64) / 16.0
+    pr = np.exp(sc - sc.max())
+    pr /= pr.sum()
+    sg = 1 / (1 + np.exp(-gate.astype(np.float64)))
+    return pr @ V * sg, pr @ np.abs(V) * sg
+
+
+def prefill(dev, desc, segs, gq, gg, T, Hq):
+    """halo_op_attn_prefill over segs [(session, start, length)], tokens in order; o fp32."""
+    arr, first = (H.PrefillSegment * len(segs))(), 0
+    for i, (s, start, n) in enumerate(segs):
+        arr[i] = H.PrefillSegment(s, start, n, first)
+        first += n
+    assert first == T
+    go = dev.array((T, Hq, D), np.float32).fill(0)
+    nbytes = H.lib().halo_op_attn_prefill_workspace_bytes(arr, len(segs))
+    ws = dev.array(nbytes, np.uint8)
+    dev.op("attn_prefill", ctypes.byref(desc), arr, len(segs), gq.ptr, gg.ptr, go.ptr, None, None, Hq, ws.ptr, nbytes)
+    return go.download()
+
+
+@pytest.mark.parametrize("T", [600, 1100, 2304])
+def test_attn_prefill_any_split_bitwise(dev, T):
+    """A prompt whole and in pieces whose tiles start at other tokens (a query then shares its wave and its 32-key
+    chunks' tiles with other queries, and the pieces take either tile size): a query's bits are its own."""
+    Hq, Hkv = 16, 2
+    rng = np.random.default_rng(T)
+    desc, g, *_ = build(dev, rng, 1, Hkv, 0, [T], T, 2.0, 1.0)
+    q = (2.0 * rng.normal(0, 1, (T, Hq, D))).astype(np.float32)
+    gate = rng.normal(0, 1, (T, Hq, D)).astype(np.float32)
+
+    def run(pieces):
+        out = []
+        for a, n in pieces:
+            gq, gg = dev.to_device(q[a : a + n]), dev.to_device(gate[a : a + n])
+            out.append(prefill(dev, desc, [(0, a, n)], gq, gg, n, Hq))
+        return np.concatenate(out).view(np.uint32)
+
+    whole = run([(0, T)])
+    for pieces in ([(0, 66), (66, 1), (67, T - 67)], [(0, 5), (5, 258), (263, T - 263)]):
+        assert np.array_equal(whole, run(pieces)), pieces
