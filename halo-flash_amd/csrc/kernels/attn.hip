@@ -699,7 +699,7 @@ extern "C" __global__ void __launch_bounds__(64)
 // Every fp32 operand x enters as a pair of halves, hi = fp16(x) and lo = fp16(x - hi) (|x - hi - lo| <= 2^-22 |x|
 // for normal values), and each product is formed as hi * hi + hi * lo + lo * hi on v_mfma_f32_32x32x16_f16
 // (products of halves are exact in the fp32 accumulator; the dropped lo * lo term is below 2^-22 of the product).
-// q, K and V are scaled by 2^8 and the probabilities by 2^10 before the split (kSqk, kSvv, kSppT); a query row, K chunk
+// q, K and V are scaled by 2^8 and the probabilities by 2^14 before the split (kSqk, kSvv, kSpp); a query row, K chunk
 // or V chunk whose magnitude would overflow fp16 at 2^8 takes a smaller power of two (halo::SplitScale), so any finite
 // operand range is accepted.
 //
@@ -731,8 +731,11 @@ extern "C" __global__ void __launch_bounds__(64)
 namespace {
 constexpr int kHalf = kChunk * kHd * 2;          // bytes of one staged matrix's hi (or lo) halves
 constexpr int kBuf = 2 * kHalf;                  // bytes of one staged chunk of K or V
-constexpr float kSppT = 1024.0f;                 // probabilities, <= 2^kLazy
-constexpr float kLazy = 5.0f;                    // the running max may lag by this (base 2) before a rescale
+// The running max may lag by this (base 2) before a rescale: probabilities up to 2^1.9 stay below 65504 at 2^14 (kSpp), the
+// scale that keeps 2^-39 of the row's largest. (2^10 with a lag of 5 saves the rescaling, 4% of an 8192-token prompt,
+// but a probability 2^20 below the largest then has an error of up to 4e-5 of itself.)
+constexpr float kLazy = 1.9f;
+static_assert(kSpp == 16384.0f);
 typedef float V16F __attribute__((ext_vector_type(16)));
 typedef short S4 __attribute__((ext_vector_type(4)));
 
@@ -843,7 +846,7 @@ __device__ __forceinline__ void AttnPrefill(
   load(kpool, pg0, 0, kraw);
   load(vpool, pg0, 0, vraw);
   const std::uint32_t qpos = p0 + tok0 + n / 8;
-  float sva = kSvv, ps = kSppT;  // V's scale in acc (the smallest so far), and the scale of P that matches it
+  float sva = kSvv, ps = kSpp;  // V's scale in acc (the smallest so far), and the scale of P that matches it
   float m = -INFINITY, l = 0.0f;
   V16F acc[NJ / 2];
 #pragma unroll
@@ -944,9 +947,9 @@ __device__ __forceinline__ void AttnPrefill(
       const float svc = fl & 2u ? restage(vpool, i, true, b, kSvv) : kSvv;
       vfac = svc < sva ? svc / sva : 1.0f;
       sva = fminf(sva, svc);
-      ps = kSppT * (sva / svc);
+      ps = kSpp * (sva / svc);
     } else {
-      ps = kSppT * (sva / kSvv);
+      ps = kSpp * (sva / kSvv);
     }
     // the running max (base-2 units) lags by up to kLazy, so few chunks rescale; a query's own scores decide when its max
     // moves, so its bits do not depend on the queries that share its wave
@@ -1069,7 +1072,7 @@ __device__ __forceinline__ void AttnPrefill(
   // epilogue: this lane's query, dims d0 + 32 c + 8 g + 4 h + e (slot 4 g + e)
   l += __shfl_xor(l, 32);
   const bool live = tok0 + n / 8 < ntok;
-  const float inv = 1.0f / l * (1.0f / (kSppT * sva));
+  const float inv = 1.0f / l * (1.0f / (kSpp * sva));
 #pragma unroll
   for (int c = 0; c < NJ / 2; ++c) {
     float v[16], amax = 0.0f;

@@ -224,7 +224,7 @@ typedef struct halo_paged_kv {
 
 /* Arithmetic: one session runs fp32 dot products; two or more sessions (and the prefill below) run the products on
  * split-fp16 matrix cores (each operand as hi + lo halves after a power-of-two scaling: q, k and V by 2^8, the
- * probabilities by 2^14, in the prefill by 2^10), within 2^-22 of each product for operands of magnitude about 1e-4 to 255. A query row, K
+ * probabilities by 2^14), within 2^-22 of each product for operands of magnitude about 1e-4 to 255. A query row, K
  * chunk or V chunk holding a magnitude of 255.875 or more takes a smaller power-of-two scale (largest value below
  * 2^15), so no finite operand overflows; that group's small values then keep a coarser absolute precision. */
 /* Scratch for the partials of one decode attention call. */

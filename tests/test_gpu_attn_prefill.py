@@ -177,3 +177,41 @@ def test_attn_prefill_any_split_bitwise(dev, T):
     whole = run([(0, T)])
     for pieces in ([(0, 66), (66, 1), (67, T - 67)], [(0, 5), (5, 258), (263, T - 263)]):
         assert np.array_equal(whole, run(pieces)), pieces
+
+
+@pytest.mark.parametrize("T", [300, 2400])  # 8-token tiles, 16-token tiles
+@pytest.mark.parametrize("bits", [8, 20])
+def test_attn_prefill_dominant_key(dev, T, bits):
+    """The first key takes the weight (2^bits above every other one) and its V is zero, so the output is made of small
+    probabilities alone. The other keys' scores are equal and V is positive, so that their rounding errors add up instead
+    of averaging out. A probability is split at 2^14 times its size against the row's largest: its low half is within
+    2^-25, 2^-39 of the largest, here at most 2^(bits + 1.5 - 39) of a probability (5.4e-6), under the 1e-5 bar."""
+    dominant_key_case(dev, T, bits)
+
+
+def dominant_key_case(dev, T, bits, outlier=None):
+    Hq, Hkv = 16, 2
+    rng = np.random.default_rng(bits)
+
+    def tweak(kp, vp, pages):
+        kp[:] = 0
+        kp[pages[0, 0], :, 0] = np.where(np.arange(D) % 3 == 0, -0.875, 0.875)
+        vp[:] = rng.uniform(0.5, 1.5, vp.shape)
+        vp[pages[0, 0], :, 0] = 0
+        if outlier is not None:
+            pos, value = outlier
+            vp[pages[0, pos // 16], :, pos % 16, 77] = value
+
+    desc, g, kp, vp, pages, _ = build(dev, rng, 1, Hkv, 0, [T], -(-T // 16) * 16, tweak=tweak)
+    # q . k0 / 16 = 14 c: the first score is bits + (0 .. 1.5) base-2 units above the others, c in steps of 2^-10 (exact)
+    c = np.round(1024 * (bits + 1.5 * rng.random((T, Hq, 1))) * np.log(2) / 14) / 1024
+    q = (c * np.where(np.arange(D) % 3 == 0, -1.0, 1.0)).astype(np.float32)
+    gate = rng.normal(0, 1, (T, Hq, D)).astype(np.float32)
+    got = prefill(dev, desc, [(0, 0, T)], dev.to_device(q), dev.to_device(gate), T, Hq)
+    assert np.isfinite(got).all()
+    worst = 0.0
+    for p in sorted({1, 31, 32, 63, 64, 100, T // 2, T - 2, T - 1} | set(rng.integers(1, T, 20).tolist())):
+        for h in range(0, Hq, 3):
+            want, mag = reference(q[p, h], gate[p, h], kp, vp, pages[0], p, h)
+            worst = max(worst, float(np.max(np.abs(got[p, h] - want) / mag)))
+    assert worst <= 1e-5, f"{worst:.3g} of sum |p| |v|"
