@@ -701,7 +701,7 @@ extern "C" __global__ void __launch_bounds__(64)
 // (products of halves are exact in the fp32 accumulator; the dropped lo * lo term is below 2^-22 of the product).
 // q, K and V are scaled by 2^8 and the probabilities by 2^14 before the split (kSqk, kSvv, kSpp); a query row, K chunk
 // or V chunk whose magnitude would overflow fp16 at 2^8 takes a smaller power of two (halo::SplitScale), so any finite
-// operand range is accepted.
+// operand range is accepted; V keeps the smallest scale from there on.
 //
 // Block (tile, kv head): 128 queries = 16 tokens x 8 q heads; wave w the tokens 4 w .. 4 w + 3, query n = 8 (token -
 // 4 w) + head. Both products run transposed, so that a query is a column and stays in one lane pair (n, n + 32)
@@ -712,7 +712,7 @@ extern "C" __global__ void __launch_bounds__(64)
 //
 // 32-key chunks, double-buffered in LDS as halves (K and V, hi and lo, [key][256]: 128 KB); one barrier per chunk: while
 // chunk i's softmax and P V run, the scores of chunk i + 1 are formed, chunk i + 2 of K and i + 1 of V are converted
-// into the buffers that became free, and the next raw chunks are on their way into registers. Overflow of the default
+// into the buffers that became free, and the next raw chunks are on their way into registers. Overflow of the
 // operand scale is flagged while converting; the flag is read after the barrier that publishes the chunk, and a flagged
 // chunk (outliers) is staged again with its own scale by the whole block.
 //
@@ -783,7 +783,7 @@ __device__ __forceinline__ void AttnPrefill(
   // in four different 32-byte bank groups)
   __shared__ __attribute__((aligned(1024))) char lds[4 * kBuf];  // K buffers 0, 1, V buffers 0, 1: hi then lo halves
   __shared__ float red[4];
-  __shared__ __attribute__((aligned(16))) std::uint32_t flags[2][2][4];  // [buffer][K, V][wave]: default scale overflowed
+  __shared__ __attribute__((aligned(16))) std::uint32_t flags[2][2][4];  // [buffer][K, V][wave]: the scale overflowed
   const std::uint32_t* tl = tiles + 4 * static_cast<std::size_t>(blockIdx.x / Hkv);
   const std::uint32_t first = tl[0], ntok = tl[1], sess = tl[2], p0 = tl[3];
   const std::uint32_t kvh = blockIdx.x % Hkv;
@@ -846,7 +846,7 @@ __device__ __forceinline__ void AttnPrefill(
   load(kpool, pg0, 0, kraw);
   load(vpool, pg0, 0, vraw);
   const std::uint32_t qpos = p0 + tok0 + n / 8;
-  float sva = kSvv, ps = kSpp;  // V's scale in acc (the smallest so far), and the scale of P that matches it
+  float sva = kSvv;  // V's scale (uniform): the smallest of the chunks so far, at which acc stands and V is staged
   float m = -INFINITY, l = 0.0f;
   V16F acc[NJ / 2];
 #pragma unroll
@@ -856,7 +856,7 @@ __device__ __forceinline__ void AttnPrefill(
   }
 
   // a chunk of K or V from registers into buffer b at the default scale, flagged by the waves where that overflows (every
-  // lane of a wave stores the same word: a store under a branch would cut the schedule)
+  // lane of a wave stores the same word: a store under a branch would cut the schedule); the prologue's chunks
   const auto stage = [&](int which, const float4 (&r)[8], std::uint32_t b) {
     flags[b ^ which][which][wave] = __any(MaxAbs(r) * 256.0f >= 65504.0f) ? 1u : 0u;
     StageRow(r, lds, (which ? vsa : ksa) + b * kBuf, 256.0f);
@@ -869,7 +869,9 @@ __device__ __forceinline__ void AttnPrefill(
     return __builtin_amdgcn_readfirstlane(w);
   };
   static_assert(kSqk == 256.0f && kSvv == 256.0f);
-  // a flagged chunk again, by the whole block, at the scale of its largest magnitude; returns the scale
+  // a flagged chunk again, by the whole block, at the scale of its largest magnitude; returns the scale, below the
+  // one that overflowed (not above it either where the magnitude is infinite and has no scale: one infinite V then
+  // spoils its own dim alone)
   const auto restage = [&](const float* pool, std::uint32_t c, bool is_v, std::uint32_t b, float base) {
     const float4* src = row(pool, pt[position(c) / kPage], c);
     float w = 0.0f;
@@ -881,7 +883,8 @@ __device__ __forceinline__ void AttnPrefill(
     w = halo::GroupMax(w);
     if (lane == 0) red[wave] = w;
     __syncthreads();
-    const float s = halo::SplitScale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])), base);
+    const float s = __uint_as_float(__builtin_amdgcn_readfirstlane(
+        __float_as_uint(fminf(base, halo::SplitScale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])), base)))));
     const std::uint32_t a0 = (is_v ? vsa : ksa) + b * kBuf;
 #pragma unroll 1
     for (int j = 0; j < 4; ++j) {
@@ -944,12 +947,11 @@ __device__ __forceinline__ void AttnPrefill(
     const std::uint32_t fl = flagged(nb);
     if (fl != 0u) {
       if (fl & 1u) fn = fq / restage(kpool, i + 1, false, nb, kSqk);
-      const float svc = fl & 2u ? restage(vpool, i, true, b, kSvv) : kSvv;
-      vfac = svc < sva ? svc / sva : 1.0f;
-      sva = fminf(sva, svc);
-      ps = kSpp * (sva / svc);
-    } else {
-      ps = kSpp * (sva / kSvv);
+      if (fl & 2u) {
+        const float svc = restage(vpool, i, true, b, sva);
+        vfac = svc / sva;
+        sva = svc;
+      }
     }
     // the running max (base-2 units) lags by up to kLazy, so few chunks rescale; a query's own scores decide when its max
     // moves, so its bits do not depend on the queries that share its wave
@@ -984,18 +986,20 @@ __device__ __forceinline__ void AttnPrefill(
         e[2 * p] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * p], f, -m));
         e[2 * p + 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * p + 1], f, -m));
       } else if (k % 3 == 1) {
-        halo::SplitPair(e[2 * p], e[2 * p + 1], ps, pw[p], pw[8 + p]);
+        halo::SplitPair(e[2 * p], e[2 * p + 1], kSpp, pw[p], pw[8 + p]);
       } else {
         ls += e[2 * p] + e[2 * p + 1];
       }
     };
     // k < 24: as stage(which, buf), in four pieces: its splits, its two stores, and the same piece of the chunk after into
-    // the registers that became free (in flight for a whole iteration)
+    // the registers that became free (in flight for a whole iteration). V at the smallest scale so far, so that P and acc
+    // need no factor of their own: a small P has no bits to spare, V loses only what the outlier's fp32 sum would
     const auto stage_slice = [&](int k, int which, float4 (&r)[8], const float4* next, std::uint32_t buf, float& top) {
       const int j = k / 6, e = k % 6;
+      const float scale = which ? sva : kSqk;
       if (e < 4) {
         const float4 x = r[2 * j + e / 2];
-        halo::SplitPair(e % 2 ? x.z : x.x, e % 2 ? x.w : x.y, 256.0f, sw[e], sw[4 + e]);
+        halo::SplitPair(e % 2 ? x.z : x.x, e % 2 ? x.w : x.y, scale, sw[e], sw[4 + e]);
         if (e % 2 == 0) top = fmaxf(top, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
       } else if (e == 4) {
         char* at = lds + (((which ? vsa : ksa) + buf * kBuf) ^ (128u * (j & 1))) + 256 * (j / 2);
@@ -1004,7 +1008,7 @@ __device__ __forceinline__ void AttnPrefill(
       } else {
         r[2 * j] = next[2 * (spart + 8 * j)];
         r[2 * j + 1] = next[2 * (spart + 8 * j) + 1];
-        if (j == 3) flags[buf ^ which][which][wave] = __any(top * 256.0f >= 65504.0f) ? 1u : 0u;
+        if (j == 3) flags[buf ^ which][which][wave] = __any(top * scale >= 65504.0f) ? 1u : 0u;
       }
     };
     // k < 24: the masked scores of chunk i + 1 and their max (from slice 4 on: the last score product has landed)

@@ -226,7 +226,8 @@ typedef struct halo_paged_kv {
  * split-fp16 matrix cores (each operand as hi + lo halves after a power-of-two scaling: q, k and V by 2^8, the
  * probabilities by 2^14), within 2^-22 of each product for operands of magnitude about 1e-4 to 255. A query row, K
  * chunk or V chunk holding a magnitude of 255.875 or more takes a smaller power-of-two scale (largest value below
- * 2^15), so no finite operand overflows; that group's small values then keep a coarser absolute precision. */
+ * 2^15), so no finite operand overflows; that group's small values then keep a coarser absolute precision (in the prefill
+ * also V's of the chunks after it, which are staged at the smallest scale so far). */
 /* Scratch for the partials of one decode attention call. */
 size_t halo_op_attn_decode_workspace_bytes(const halo_paged_kv* kv, uint32_t q_heads);
 /* o [S][Hq][d] = attention(q [S][Hq][d]) over each session's nkv positions; gate [S][Hq][d] or NULL. Two launches. */

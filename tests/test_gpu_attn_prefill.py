@@ -215,3 +215,70 @@ def dominant_key_case(dev, T, bits, outlier=None):
             want, mag = reference(q[p, h], gate[p, h], kp, vp, pages[0], p, h)
             worst = max(worst, float(np.max(np.abs(got[p, h] - want) / mag)))
     assert worst <= 1e-5, f"{worst:.3g} of sum |p| |v|"
+
+
+@pytest.mark.parametrize("T", [300, 2400])  # 8-token tiles, 16-token tiles
+@pytest.mark.parametrize("outlier", [(5, 1e6), (40, 1e6), (40, 1e4), (270, -1e6)])
+def test_attn_prefill_value_outlier(dev, T, outlier):
+    """One V far above the rest (position, value), in the first 32-key chunk, the second or a later one: V of the chunks
+    after it is staged at its smaller scale (2^-5 for 1e6: V keeps 2^-20 of itself) and the accumulators before it are
+    rescaled exactly, while the probabilities, 2^8 below the first key's, keep their bits; the 1e-5 bar in every dim."""
+    dominant_key_case(dev, T, 8, outlier)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_attn_prefill_nonfinite_value(dev, value):
+    """An infinite or NaN V makes its own dim of the queries that see its chunk non-finite, and nothing else."""
+    Hq, Hkv, T, pos = 16, 2, 200, 70
+    rng = np.random.default_rng(3)
+    tweak = lambda kp, vp, pages: vp[pages[0, pos // 16]].__setitem__((slice(None), pos % 16, 9), value)  # noqa: E731
+    desc, g, kp, vp, pages, _ = build(dev, rng, 1, Hkv, 0, [T], 208, tweak=tweak)
+    q, gate = (rng.normal(0, 1, (T, Hq, D)).astype(np.float32) for _ in range(2))
+    got = prefill(dev, desc, [(0, 0, T)], dev.to_device(q), dev.to_device(gate), T, Hq)
+    others = np.arange(D) != 9
+    assert np.isfinite(got[..., others]).all() and np.isfinite(got[:64]).all()
+    assert not np.isfinite(got[pos:, :, 9]).any()
+    vp[pages[0, pos // 16], :, pos % 16, 9] = 0
+    for p in (63, 69, 70, 95, 96, T - 1):
+        want, mag = reference(q[p, 3], gate[p, 3], kp, vp, pages[0], p, 3)
+        assert np.all((np.abs(got[p, 3] - want) <= 1e-5 * mag + 1e-6)[others])
+
+
+@pytest.mark.parametrize("qk,v,outliers", [(1.0, 1.0, False), (0.1, 1e-3, False), (2.0, 50.0, False), (1.0, 1.0, True)])
+def test_attn_prefill_long_segments(dev, qk, v, outliers):
+    """Ragged segments behind a shared prefix, long enough for 16-token tiles: plain, small and large operands, and outlier
+    channels (V's on the page of positions 32 .. 47 of the prefix alone), as the short cases above, against 64 bits at
+    tokens around tile, chunk and segment edges and at random ones; the Q8 output is the fp32 output's."""
+    Hq, Hkv, prefix = 16, 2, 512
+    segs = [(0, 512, 700), (1, 512, 1100), (2, 512, 1), (3, 512, 513)]
+    rng = np.random.default_rng(int(10 * v) + outliers)
+    tweak = (lambda k_, v_, p_: outlier_kv(k_, v_, v_pages=[int(p_[0, 2])])) if outliers else None
+    desc, g, kp, vp, pages, _ = build(dev, rng, 4, Hkv, prefix, [1100] * 4, 1616, qk, v, tweak=tweak)
+    T = sum(n for *_, n in segs)
+    q = (qk * rng.normal(0, 1, (T, Hq, D))).astype(np.float32)
+    if outliers:
+        outlier_q(q)
+    gate = rng.normal(0, 1, (T, Hq, D)).astype(np.float32)
+    gq, gg = dev.to_device(q), dev.to_device(gate)
+    arr, first = (H.PrefillSegment * 4)(), 0
+    for i, (s, start, n) in enumerate(segs):
+        arr[i] = H.PrefillSegment(s, start, n, first)
+        first += n
+    go, goq = dev.array((T, Hq, D), np.float32), dev.array((T, Hq * D), np.int8)
+    gos = dev.array((T, Hq * D // 32), np.float32)
+    nbytes = H.lib().halo_op_attn_prefill_workspace_bytes(arr, 4)
+    ws = dev.array(nbytes, np.uint8)
+    dev.op("attn_prefill", ctypes.byref(desc), arr, 4, gq.ptr, gg.ptr, go.ptr, goq.ptr, gos.ptr, Hq, ws.ptr, nbytes)
+    got = go.download()
+    assert np.isfinite(got).all()
+    first = 0
+    for s, start, n in segs:
+        picks = {0, 1, 7, 8, 15, 16, 31, 32, n - 2, n - 1} | set(rng.integers(0, n, 12).tolist())
+        for k in sorted(x for x in picks if 0 <= x < n):
+            for h in range(Hq):
+                want, mag = reference(q[first + k, h], gate[first + k, h], kp, vp, pages[s], start + k, h)
+                assert np.all(np.abs(got[first + k, h] - want) <= 1e-5 * mag), f"session {s} position {start + k} head {h}"
+        first += n
+    xq, xs = O.quantize(got.reshape(T, Hq * D))
+    assert np.array_equal(goq.download(), xq)
+    assert np.array_equal(gos.download().view(np.uint32), xs.view(np.uint32))
