@@ -9,6 +9,8 @@
 // chunk is read once and scored against the queries of every session (S * G query vectors), a suffix chunk only
 // against its own session's G queries. Each (kv head, 32-token chunk) is one block producing flash partials
 // (running max, sum, weighted V); halo_attn_decode_combine merges them per (session, head) and applies the gate.
+#include <type_traits>
+
 #include "common.h"
 
 using halo::kWave;
@@ -722,7 +724,10 @@ extern "C" __global__ void __launch_bounds__(64)
 // the conversions per query. One wave per SIMD hides nothing by itself, hence the hand-placed slices of vector work after each
 // matrix instruction. Registers: accumulators and most of Q in AGPRs (pinned; otherwise the compiler moves all 128
 // accumulators through VGPRs each chunk), no scratch.
-// One 8192-token prompt, 16 heads (550 GFLOP of fp32 products): 3.70 -> 1.70 ms = 323 TFLOP/s (970 of fp16 MFMA issue; a
+// One block per CU also means that nothing covers a block's ends: the query row and the first chunk are loaded in one
+// round trip, the gate's values in another, and the last chunk forms no further scores (20 tokens 33 -> 28 us a call, 512
+// tokens 70 -> 65, 400 prompts of 20 tokens 237 -> 168).
+// One 8192-token prompt, 16 heads (550 GFLOP of fp32 products): 3.70 -> 1.73 ms = 318 TFLOP/s (955 of fp16 MFMA issue; a
 // large library bf16 matrix product reaches 1380 on this card). The form before held 16 queries per wave, 8 tokens per
 // block, with P through LDS.
 // AttnPrefill<2> (halo_attn_prefill_d2): 8-token tiles, two waves share 32 queries and split the output dims: 0.75x the
@@ -815,39 +820,43 @@ __device__ __forceinline__ void AttnPrefill(
     }
   };
   std::uint32_t pg0 = pt[position(0) / kPage], pg1 = pt[position(1) / kPage], pg2 = pt[position(2) / kPage];
-  // this lane's query: dims 16 c + 8 h .. + 7 of step c (the B operand)
+  __builtin_amdgcn_sched_barrier(0);
+  // this lane's query: dims 16 c + 8 h .. + 7 of step c (the B operand). Its whole row and the first chunk are in flight
+  // together (read in two passes, the second a few values at a time, the row took longer than a short prompt's products)
   const std::uint32_t tok = min(tok0 + n / 8, ntok - 1);
   const std::size_t qbase = ((static_cast<std::size_t>(first) + tok) * Hq + kvh * 8 + n % 8) * kHd;
   H8 qh[kHd / 16], ql[kHd / 16];
   float fq;
   {
     const float* qrow = q + qbase + 8 * h;
+    float4 x4[kHd / 8];
     float amax = 0.0f;
 #pragma unroll
-    for (int c = 0; c < kHd / 16; ++c) {
-      const float4 a = *reinterpret_cast<const float4*>(qrow + 16 * c), b = *reinterpret_cast<const float4*>(qrow + 16 * c + 4);
-      amax = fmaxf(amax, fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
-                               fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w)))));
-    }
+    for (int c = 0; c < kHd / 8; ++c) x4[c] = *reinterpret_cast<const float4*>(qrow + 16 * (c / 2) + 4 * (c % 2));
+    __builtin_amdgcn_sched_barrier(0);
+    load(kpool, pg0, 0, kraw);
+    load(vpool, pg0, 0, vraw);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < kHd / 8; ++c)
+      amax = fmaxf(amax, fmaxf(fmaxf(fabsf(x4[c].x), fabsf(x4[c].y)), fmaxf(fabsf(x4[c].z), fabsf(x4[c].w))));
     amax = fmaxf(amax, __shfl_xor(amax, 32));
     const float sq = halo::SplitScale(amax, kSqk);
 #pragma unroll
-    for (int c = 0; c < kHd / 16; ++c) {  // (read again: the row is in the cache, and 128 floats need no registers)
-      const float4 a = *reinterpret_cast<const float4*>(qrow + 16 * c), b = *reinterpret_cast<const float4*>(qrow + 16 * c + 4);
+    for (int c = 0; c < kHd / 16; ++c) {
+      const float4 a = x4[2 * c], b = x4[2 * c + 1];
       const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
       SplitHalves(x, qh[c], ql[c], sq);
-      __builtin_amdgcn_sched_barrier(0);  // a few of the row's loads at a time
+      __builtin_amdgcn_sched_barrier(0);
       asm("" : "+a"(qh[c]));
       if (c < 8) asm("" : "+a"(ql[c]));
     }
     // scores and the running max in base-2 units: each exponential is one v_exp_f32
     fq = (1.0f / sqrtf(static_cast<float>(kHd))) * kLog2e / sq;
   }
-  load(kpool, pg0, 0, kraw);
-  load(vpool, pg0, 0, vraw);
   const std::uint32_t qpos = p0 + tok0 + n / 8;
   float sva = kSvv;  // V's scale (uniform): the smallest of the chunks so far, at which acc stands and V is staged
-  float m = -INFINITY, l = 0.0f;
+  float l = 0.0f;
   V16F acc[NJ / 2];
 #pragma unroll
   for (int c = 0; c < NJ / 2; ++c) {
@@ -936,17 +945,20 @@ __device__ __forceinline__ void AttnPrefill(
     cm = fmaxf(cm, s[j]);
   }
   cm = pair_max(cm) * f;
+  float m = cm;
   stage(0, kraw, 1);
   load(kpool, pg2, 2, kraw);
   pg1 = pg2;  // at iteration i: pg1, pg2 the pages of chunks i + 2, i + 3
   pg2 = pt[position(3) / kPage];
-  for (std::uint32_t i = 0; i < nchunks; ++i) {
+  // chunk i; the last one has no scores to form and nothing to stage (a third of a one-chunk block's products)
+  const auto step = [&](auto is_last, std::uint32_t i) __attribute__((always_inline)) {
+    constexpr bool kLast = is_last;
     const std::uint32_t b = i & 1, nb = b ^ 1;
     halo::LdsSync();  // K of chunk i + 1 and V of chunk i are staged; the buffers of K i and V i - 1 are free
     float fn = fq / kSqk, vfac = 1.0f;  // score factor of chunk i + 1 (exact: the scales are powers of two)
     const std::uint32_t fl = flagged(nb);
     if (fl != 0u) {
-      if (fl & 1u) fn = fq / restage(kpool, i + 1, false, nb, kSqk);
+      if (!kLast && (fl & 1u)) fn = fq / restage(kpool, i + 1, false, nb, kSqk);
       if (fl & 2u) {
         const float svc = restage(vpool, i, true, b, sva);
         vfac = svc / sva;
@@ -972,8 +984,8 @@ __device__ __forceinline__ void AttnPrefill(
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    // P^T of chunk i (slots 8 st .. 8 st + 7 are the k order of step st) beside the scores of chunk i + 1 (past the end:
-    // the clamped chunk's, unused), then P V beside the conversions: after each matrix instruction a slice of the vector
+    // P^T of chunk i (slots 8 st .. 8 st + 7 are the k order of step st) beside the scores of chunk i + 1,
+    // then P V beside the conversions: after each matrix instruction a slice of the vector
     // work that it hides (the barriers keep that order), each step's fragments read one step ahead.
     H8 ah[2], al[2];
     V16F sn = {};
@@ -1022,33 +1034,39 @@ __device__ __forceinline__ void AttnPrefill(
       }
     };
     const float4 *knext = nullptr, *vnext = nullptr;
-    kfrag(nb, 0, ah[0], al[0]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 0; k < 9; ++k) softmax_slice(k);  // while the first fragments arrive
-    __builtin_amdgcn_sched_barrier(0);
     float top = 0.0f;
+    if constexpr (!kLast) {
+      kfrag(nb, 0, ah[0], al[0]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      if (c < 15)
-        kfrag(nb, c + 1, ah[(c + 1) % 2], al[(c + 1) % 2]);
-      else
-        vfrag(b, 0, ah[0], al[0]);
+      for (int k = 0; k < 9; ++k) softmax_slice(k);  // while the first fragments arrive
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int p = 0; p < 3; ++p) {
-        sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(p == 0 ? al[c % 2] : ah[c % 2], p == 1 ? ql[c] : qh[c], sn, 0, 0, 0);
-        if (c == 0 && p == 1) {
-          knext = row(kpool, pg2, i + 3);
-          vnext = row(vpool, pg1, i + 2);
-          pg1 = pg2;
-          pg2 = pt[position(i + 4) / kPage];  // ahead of this iteration's row loads: not waited for with them
-        }
-        if (c < 8)
-          softmax_slice(3 * c + p + 9 < 24 ? 3 * c + p + 9 : 24);
+      for (int c = 0; c < 16; ++c) {
+        if (c < 15)
+          kfrag(nb, c + 1, ah[(c + 1) % 2], al[(c + 1) % 2]);
         else
-          stage_slice(3 * (c - 8) + p, 0, kraw, knext, b, top);
-        __builtin_amdgcn_sched_barrier(0);
+          vfrag(b, 0, ah[0], al[0]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          sn = __builtin_amdgcn_mfma_f32_32x32x16_f16(p == 0 ? al[c % 2] : ah[c % 2], p == 1 ? ql[c] : qh[c], sn, 0, 0, 0);
+          if (c == 0 && p == 1) {
+            knext = row(kpool, pg2, i + 3);
+            vnext = row(vpool, pg1, i + 2);
+            pg1 = pg2;
+            pg2 = pt[position(i + 4) / kPage];  // ahead of this iteration's row loads: not waited for with them
+          }
+          if (c < 8)
+            softmax_slice(3 * c + p + 9 < 24 ? 3 * c + p + 9 : 24);
+          else
+            stage_slice(3 * (c - 8) + p, 0, kraw, knext, b, top);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
+    } else {
+      vfrag(b, 0, ah[0], al[0]);
+#pragma unroll
+      for (int k = 0; k < 24; ++k) softmax_slice(k);
     }
     l += ls;
     cm = -INFINITY;
@@ -1066,14 +1084,22 @@ __device__ __forceinline__ void AttnPrefill(
       for (int p = 0; p < 3; ++p) {
         acc[j / 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(p == 0 ? al[j % 2] : ah[j % 2], p == 1 ? pl[j % 2] : ph[j % 2],
                                                              acc[j / 2], 0, 0, 0);
-        if (j < 8) score_slice(3 * j + p);
-        if (j >= NJ - 8) stage_slice(3 * (j - (NJ - 8)) + p, 1, vraw, vnext, nb, top);
+        if (!kLast && j < 8) score_slice(3 * j + p);
+        if (!kLast && j >= NJ - 8) stage_slice(3 * (j - (NJ - 8)) + p, 1, vraw, vnext, nb, top);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     f = fn;
-  }
+  };
+  for (std::uint32_t i = 0; i + 1 < nchunks; ++i) step(std::false_type{}, i);
+  step(std::true_type{}, nchunks - 1);
   // epilogue: this lane's query, dims d0 + 32 c + 8 g + 4 h + e (slot 4 g + e)
+  float4 gt[NJ / 2][4];  // all in flight at once: between the branches below each would be waited for by itself
+#pragma unroll
+  for (int c = 0; c < NJ / 2; ++c)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) gt[c][g] = *reinterpret_cast<const float4*>(gate + qbase + d0 + 32 * c + 8 * g + 4 * h);
+  __builtin_amdgcn_sched_barrier(0);
   l += __shfl_xor(l, 32);
   const bool live = tok0 + n / 8 < ntok;
   const float inv = 1.0f / l * (1.0f / (kSpp * sva));
@@ -1083,11 +1109,10 @@ __device__ __forceinline__ void AttnPrefill(
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const std::size_t at = qbase + d0 + 32 * c + 8 * g + 4 * h;
-      const float4 gt = *reinterpret_cast<const float4*>(gate + at);
-      v[4 * g] = acc[c][4 * g] * inv * halo::Sigmoid(gt.x);
-      v[4 * g + 1] = acc[c][4 * g + 1] * inv * halo::Sigmoid(gt.y);
-      v[4 * g + 2] = acc[c][4 * g + 2] * inv * halo::Sigmoid(gt.z);
-      v[4 * g + 3] = acc[c][4 * g + 3] * inv * halo::Sigmoid(gt.w);
+      v[4 * g] = acc[c][4 * g] * inv * halo::Sigmoid(gt[c][g].x);
+      v[4 * g + 1] = acc[c][4 * g + 1] * inv * halo::Sigmoid(gt[c][g].y);
+      v[4 * g + 2] = acc[c][4 * g + 2] * inv * halo::Sigmoid(gt[c][g].z);
+      v[4 * g + 3] = acc[c][4 * g + 3] * inv * halo::Sigmoid(gt[c][g].w);
       if (live && o != nullptr) *reinterpret_cast<float4*>(o + at) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(v[4 * g + e]));
