@@ -33,6 +33,50 @@ void Chunks(const halo_paged_kv* kv, std::uint32_t* prefix_chunks, std::uint32_t
   *suffix_chunks = std::max<std::uint32_t>(1, CeilDiv(kv->max_context - kv->prefix, kChunk));
 }
 
+// ---- prefill tiles ---------------------------------------------------------------------------------------------------
+// Two tile sizes with the same bits (halo_attn_prefill: 16 tokens a block; halo_attn_prefill_d2: 8). Which one is faster
+// depends on how the batch's blocks, one per CU, fill the 256 CUs. A block's time in hundredths of a 16-token block's
+// 32-key chunk (2.7 us), fitted to calls of 20 to 8192 tokens:
+constexpr std::uint64_t kCUs = 256;
+std::uint64_t TileTime(std::uint32_t tile, std::uint64_t end) {
+  return tile == 8 ? 600 + 84 * CeilDiv(end, kChunk) : 800 + 100 * CeilDiv(end, kChunk);
+}
+
+using Tile = std::array<std::uint32_t, 4>;  // first token in the batch, tokens, session, position of the first
+
+// Longest first: a block's work grows with its tile's position, and blocks start in grid order.
+std::vector<Tile> PrefillTiles(const halo_prefill_segment* segs, std::uint32_t nseg, std::uint32_t tile) {
+  std::vector<Tile> tiles;
+  for (std::uint32_t i = 0; i < nseg; ++i) {
+    const halo_prefill_segment& g = segs[i];
+    for (std::uint32_t k = CeilDiv(g.length, tile) * tile; k > 0; k -= tile)
+      tiles.push_back({g.first + k - tile, std::min(tile, g.length - (k - tile)), g.session, g.start + k - tile});
+  }
+  const auto longer = [](const Tile& a, const Tile& b) { return a[3] + a[1] > b[3] + b[1]; };
+  if (!std::is_sorted(tiles.begin(), tiles.end(), longer)) std::stable_sort(tiles.begin(), tiles.end(), longer);
+  return tiles;
+}
+
+// The blocks' time spread evenly over the CUs, 15% longer where that is what binds (all CUs busy clock lower, and blocks
+// go to the XCDs in turn, not to the first free CU).
+std::uint64_t EvenTime(const halo_prefill_segment* segs, std::uint32_t nseg, std::uint32_t tile, std::uint32_t heads) {
+  std::uint64_t sum = 0;
+  for (std::uint32_t i = 0; i < nseg; ++i)
+    for (std::uint32_t k = 0; k < segs[i].length; k += tile)
+      sum += TileTime(tile, segs[i].start + std::min(k + tile, segs[i].length));
+  return sum * heads * 115 / 100 / kCUs;
+}
+
+// The batch's time: even, or k + 1 blocks at least as long as block 256 k (longest first) one after the other on some CU.
+std::uint64_t BatchTime(const std::vector<Tile>& tiles, std::uint32_t tile, std::uint64_t even, std::uint32_t heads) {
+  std::uint64_t t = even;
+  for (std::uint64_t k = 0; kCUs * k < tiles.size() * heads; ++k) {
+    const Tile& x = tiles[kCUs * k / heads];
+    t = std::max(t, (k + 1) * TileTime(tile, std::uint64_t{x[3]} + x[1]));
+  }
+  return t;
+}
+
 }  // namespace
 
 extern "C" {
@@ -138,30 +182,38 @@ int halo_op_attn_prefill(halo_engine* eng, const halo_paged_kv* kv, const halo_p
   if (segs == nullptr || nseg == 0 || q == nullptr || gate == nullptr || (o == nullptr && oq == nullptr) ||
       ((oq == nullptr) != (os == nullptr)))
     return SetErr(err, errlen, "attn prefill: missing arguments"), -1;
-  // 16-token tiles, or 8-token ones (the output dims split over two waves) where those still fit the 256 CUs once
-  std::uint64_t tiles8 = 0;
-  for (std::uint32_t i = 0; i < nseg; ++i) tiles8 += CeilDiv(segs[i].length, 8);
-  const std::uint32_t tile = tiles8 * kv->kv_heads <= 256 ? 8 : 16;
-  std::vector<std::array<std::uint32_t, 4>> tiles;
+  std::size_t tiles8 = 0;
   for (std::uint32_t i = 0; i < nseg; ++i) {
     const halo_prefill_segment& g = segs[i];
-    if (g.session >= kv->sessions || g.length == 0 || g.start + g.length > kv->max_context)
+    if (g.session >= kv->sessions || g.length == 0 || std::uint64_t{g.start} + g.length > kv->max_context)
       return SetErr(err, errlen, "attn prefill: segment %u (session %u, %u + %u) out of range", i, g.session, g.start,
                     g.length),
              -1;
-    for (std::uint32_t k = 0; k < g.length; k += tile)
-      tiles.push_back({g.first + k, std::min<std::uint32_t>(tile, g.length - k), g.session, g.start + k});
+    tiles8 += CeilDiv(g.length, 8);
   }
-  // longest first: a block's work grows with its tile's position, and blocks start in grid order
-  std::stable_sort(tiles.begin(), tiles.end(), [](const auto& a, const auto& b) { return a[3] + a[1] > b[3] + b[1]; });
+  // The tile size that is expected to be done first (16-token tiles need the smaller workspace). Measured at 2 kv heads, in us,
+  // 8-token / 16-token tiles: one prompt of 20 tokens 28 / 33, of 512 65 / 79, 1040 102 / 126, 1800 171 / 186, 2048 208 / 208, 2400
+  // 298 / 239, 8192 2783 / 1703; 256 tokens at position 8192, 1 / 4 / 8 of them, 589 / 694, 690 / 698, 1354 / 840; at position 1000, 200 of 8
+  // tokens 193 / 228, 100 of 12 187 / 126.
+  std::uint32_t tile = 16;
+  std::vector<Tile> tiles = PrefillTiles(segs, nseg, 16);
+  const std::uint64_t t16 = BatchTime(tiles, 16, EvenTime(segs, nseg, 16, kv->kv_heads), kv->kv_heads);
+  const std::uint64_t even8 = EvenTime(segs, nseg, 8, kv->kv_heads);
+  if (even8 < t16 && ws_bytes >= tiles8 * sizeof(Tile)) {
+    std::vector<Tile> small = PrefillTiles(segs, nseg, 8);
+    if (BatchTime(small, 8, even8, kv->kv_heads) < t16) {
+      tile = 8;
+      tiles.swap(small);
+    }
+  }
   const std::size_t need = tiles.size() * sizeof(tiles[0]);
   if (ws == nullptr || ws_bytes < need) return SetErr(err, errlen, "attn prefill: workspace %zu < %zu", ws_bytes, need), -1;
   halo_buffer b{ws, need, nullptr};
   if (halo_upload(halo_engine_device(eng), &b, 0, tiles.data(), need, err, errlen) != 0) return -1;
   const halo_arg a[] = {Ptr(q), Ptr(gate), Ptr(kv->k_pool), Ptr(kv->v_pool), Ptr(kv->pages), Ptr(ws), Ptr(o), Ptr(oq),
                         Ptr(os), U32(Hq), U32(kv->kv_heads), U32(kv->max_pages)};
-  return Launch(eng, tile == 8 ? "halo_attn_prefill_d2" : "halo_attn_prefill", D3(static_cast<std::uint32_t>(tiles.size() * kv->kv_heads)), D3(256), a,
-                err, errlen);
+  return Launch(eng, tile == 8 ? "halo_attn_prefill_d2" : "halo_attn_prefill",
+                D3(static_cast<std::uint32_t>(tiles.size() * kv->kv_heads)), D3(256), a, err, errlen);
 }
 
 int halo_op_kv_append(halo_engine* eng, const halo_paged_kv* kv, const float* k, const float* v, char* err,

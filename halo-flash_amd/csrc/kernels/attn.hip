@@ -731,8 +731,8 @@ extern "C" __global__ void __launch_bounds__(64)
 // large library bf16 matrix product reaches 1380 on this card). The form before held 16 queries per wave, 8 tokens per
 // block, with P through LDS.
 // AttnPrefill<2> (halo_attn_prefill_d2): 8-token tiles, two waves share 32 queries and split the output dims: 0.75x the
-// matrix work per wave and twice the blocks, for batches whose 8-token tiles fit the 256 CUs once (256 tokens at position
-// 8192: 840 us with 16-token tiles, 734 with these, on one build of this kernel; now 581, 1167 before).
+// matrix work per wave and twice the blocks, for batches that 16-token tiles would spread unevenly over the CUs (256 tokens
+// at position 8192: 694 us with 16-token tiles, 589 with these; 1160 in the form before).
 namespace {
 constexpr int kHalf = kChunk * kHd * 2;          // bytes of one staged matrix's hi (or lo) halves
 constexpr int kBuf = 2 * kHalf;                  // bytes of one staged chunk of K or V

@@ -99,12 +99,12 @@ def test_attn_prefill_tile_edges(dev, segs):
 
 
 def test_attn_prefill_tile_shapes_bitwise(dev):
-    """A 1100-token prompt takes 16-token tiles, the same prompt in calls of 512 tokens 8-token ones (the output dims split
+    """A 2300-token prompt takes 16-token tiles, the same prompt in calls of 512 tokens 8-token ones (the output dims split
     over two waves): a query's operations are the same in both, so the outputs are equal bit for bit; and tokens at
     the edges of tiles and chunks match softmax attention in 64 bits within 1e-5 of sum |p| |v|."""
-    Hq, Hkv, T = 16, 2, 1100
+    Hq, Hkv, T = 16, 2, 2300
     rng = np.random.default_rng(11)
-    desc, g, kp, vp, pages, _ = build(dev, rng, 1, Hkv, 0, [1104], 1104, 2.0, 1.0)
+    desc, g, kp, vp, pages, _ = build(dev, rng, 1, Hkv, 0, [T], 2304, 2.0, 1.0)
     q = (2.0 * rng.normal(0, 1, (T, Hq, D))).astype(np.float32)
     gate = rng.normal(0, 1, (T, Hq, D)).astype(np.float32)
     gq, gg = dev.to_device(q), dev.to_device(gate)
@@ -120,8 +120,8 @@ def test_attn_prefill_tile_shapes_bitwise(dev):
         return go.download()
 
     whole = run([(0, T)])
-    assert np.array_equal(whole.view(np.uint32), run([(0, 512), (512, 512), (1024, 76)]).view(np.uint32))
-    for p in (0, 3, 15, 16, 31, 32, 33, 511, 1087, 1088, T - 1):
+    assert np.array_equal(whole.view(np.uint32), run([(k, min(512, T - k)) for k in range(0, T, 512)]).view(np.uint32))
+    for p in (0, 3, 15, 16, 31, 32, 33, 511, 1087, 1088, T - 2, T - 1):
         for h in (0, 7, 8, 15):
             K = gather(kp, pages[0], p + 1, h // 8).astype(np.float64)
             V = gather(vp, pages[0], p + 1, h // 8).astype(np.float64)
