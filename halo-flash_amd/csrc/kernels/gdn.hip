@@ -99,16 +99,13 @@ extern "C" __global__ void __launch_bounds__(256)
 //   Uk = T diag(beta gamma) K,  Wv = T diag(beta) V,  Qe = diag(gamma) Q - P Uk,  Ov = P Wv      (64 x 128 each)
 // and the chunk-serial part (halo_gdn_wy_scan), three products per chunk:
 //   Delta = Wv - Uk S0,  O = (Qe S0 + Ov) / sqrt(d),  S_C = gamma_C S0 + K^T diag(exp(G_C - G_s)) Delta.
-// Tokens past a partial chunk's end are zero-padded (k = q = v = 0, beta = 0, g = 0): their rows of every product are
-// zero. Inputs q, k [tokens][Hk][128] and v [tokens][Hv][128] are bf16 (the C3 operator) or fp32 (the model's
+// Tokens past a partial chunk's end have k = 0, beta = 0, g = 0 in the preparation, so their rows of Uk and Wv are zero, and
+// weight 0 in the state's update; their q and v repeat the last token's (v meets beta = 0, the rows of Qe are not used). Inputs q, k [tokens][Hk][128] and v [tokens][Hv][128] are bf16 (the C3 operator) or fp32 (the model's
 // prefill, which matches its decode step); g, beta [tokens][Hv] fp32 (g = log decay, beta after its sigmoid); state
 // fp32 [seq][Hv][128][128] key-major. chunks [n][3] = {first token, length, sequence}; seqs [n_seq][2] = {first
 // chunk, chunk count}. Workspace per (chunk, head): Uk, Qe, Wv, Ov fp32 [64][128] and the weights [64].
 namespace {
 constexpr int kC = 64;
-constexpr int kCL = 132;  // LDS row stride (floats) of a 64 x 128 tile
-constexpr int kPL = 68;   // of a 64 x 64 tile
-typedef float V16F __attribute__((ext_vector_type(16)));
 typedef float V4F __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float Bf(std::uint16_t h) { return __uint_as_float(static_cast<std::uint32_t>(h) << 16); }
@@ -122,15 +119,6 @@ struct alignas(16) Pack8 {
 template <typename In>
 __device__ __forceinline__ Pack8<In> Ld8(const In* p) {
   return *reinterpret_cast<const Pack8<In>*>(p);
-}
-// row r of a 64 x 128 LDS tile from 8 inputs: two float4 stores, zeros when !on
-template <typename In>
-__device__ __forceinline__ void Put8(float* dst, const Pack8<In>& x, bool on) {
-  float f[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) f[e] = on ? Cv(x.v[e]) : 0.0f;
-  reinterpret_cast<float4*>(dst)[0] = make_float4(f[0], f[1], f[2], f[3]);
-  reinterpret_cast<float4*>(dst)[1] = make_float4(f[4], f[5], f[6], f[7]);
 }
 }  // namespace
 
