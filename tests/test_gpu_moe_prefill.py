@@ -110,6 +110,37 @@ def test_moe_prefill_matches_oracle(dev, c2, small, shape, T):
 
 @pytest.mark.parametrize("T", [260, 560])
 def test_moe_prefill_split_groups(dev, c2, small, T):
-    """Groups a little over one tile (about 65 pairs in 64-pair tiles, 140 in 128-pair ones, the shared expert's group
-    several tiles): cut into like tiles of whole 32s, with waves past a tile's end idle."""
+    """Groups a little over one tile: about 65 pairs in 64-pair tiles (64 + 1) and 140 in 128-pair ones (96 + 44: like tiles of
+    whole 32s, a wave past a tile's end idle); the shared expert's group several tiles."""
     test_moe_prefill_matches_oracle(dev, c2, small, "small", T)
+
+
+@pytest.mark.parametrize("tile,shared", [(64, 0), (64, 1), (128, 1)])
+def test_group_scan_tiles(dev, tile, shared):
+    """The tile table itself: every group covered once and in order by tiles of at most `tile` pairs, none empty, each a
+    whole number of 32s but a group's last, and no larger than the even share rounded up to 32s."""
+    sizes = [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 156, 192, 193, 256, 257, 288, 289, 1281]
+    expect = {129: [96, 33], 156: [96, 60], 192: [96, 96], 193: [128, 65], 257: [96, 96, 65], 288: [96, 96, 96],
+              289: [128, 128, 33]} if tile == 128 else {65: [64, 1], 129: [64, 64, 1], 156: [64, 64, 28]}
+    E, T = len(sizes), 300 if shared else 0
+    parts = np.random.default_rng(tile).integers(0, np.array(sizes) + 1)  # two partial histograms
+    count = dev.to_device(np.stack([parts, np.array(sizes) - parts]).astype(np.uint32))
+    groups = sizes + [T]
+    want = sum(-(-n // tile) for n in groups)
+    start, tiles = dev.array(E + 2, np.uint32), dev.array((want, 3), np.uint32)
+    ntiles = dev.array(1, np.uint32)
+    dev.launch("halo_moe_group_scan", (1,), (1024,), [count, start, tiles, ntiles, ("u32", E), ("u32", T), ("u32", shared),
+                                                      ("u32", tile), ("u32", 2)])
+    assert int(ntiles.download()[0]) == want
+    assert start.download().tolist() == np.concatenate([[0], np.cumsum(groups)]).tolist()
+    table, row = tiles.download(), 0
+    for e, n in enumerate(groups):
+        nt, at = -(-n // tile), int(np.sum(groups[:e]))
+        mine = table[row : row + nt]
+        row += nt
+        got = mine[:, 2].tolist()
+        assert (mine[:, 0] == e).all() and mine[:, 1].tolist() == (at + np.cumsum([0] + got[:-1])).tolist()[:nt]
+        assert sum(got) == n and all(0 < x <= tile for x in got) and all(x % 32 == 0 for x in got[:-1])
+        if nt:
+            assert max(got) <= -(-(-(-n // nt)) // 32) * 32
+        assert got == expect.get(n, got)
