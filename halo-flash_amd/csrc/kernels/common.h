@@ -117,11 +117,13 @@ __device__ __forceinline__ float Group8Max(float v) {
   return fmaxf(v, Dpp<0x141>(v));
 }
 
-// Q8 codes of values that share one scale: rint(v / scale) with the bits of the IEEE division, for three instructions a value
-// instead of the eleven of a division. y = RN(1 / scale) is one division per scale; q = RN(v y) is then within an ulp of
-// v / scale, its residual v - scale q is exact in one FMA, and RN(q + residual y) is the correctly rounded quotient
-// (Markstein's theorem; checked over every mantissa of the scale at every half-integer quotient and three ulps around it). Scales
-// below 2^-60 and their values are multiplied by 2^64 first (exact), so no step underflows. A zero scale codes 0.
+// Q8 codes of values that share one scale: rint(v / scale) with the bits of the IEEE division, for four instructions a value
+// instead of the eleven of a division. y = RN(1 / scale) is one division per scale; q = RN(v y) is then within 1.5 ulps of
+// v / scale, and q + (v - scale q) y, its residual and sum one FMA each, within 2^-21 ulps before the last rounding (a step
+// of Newton's iteration, as in Markstein's division). That decides the code unless v / scale is that close to the middle between
+// two floats next to a half-integer, which no quotient is: checked for every mantissa of the scale at every half-integer
+// and the values within two ulps of it (a host test of this struct). Scales below 2^-60 and their values are multiplied by
+// 2^64 first (exact), so no step underflows. A zero scale codes 0.
 struct CodeScale {
   float up, b, y;
   __device__ __forceinline__ explicit CodeScale(float scale) {

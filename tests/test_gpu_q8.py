@@ -75,11 +75,12 @@ def test_quantizer_pair_bit_exact(dev, tokens):
         assert np.array_equal(sc.download().view(np.uint32), xs.view(np.uint32))
 
 
-def _near_tie_rows(rng, tokens, cols):
+def _near_tie_rows(rng, tokens, cols, amax=None):
     """Rows whose 32-value blocks hold an amax and 31 values within a few ulps of (k + 1/2) * scale: quotients at
     half-integers, where any quotient other than the IEEE one (a reciprocal times v) can round the other way."""
     nb = tokens * cols // 32
-    amax = (np.abs(rng.normal(0, 1, nb)) * 10.0 ** rng.integers(-6, 6, nb) + 1e-3).astype(np.float32)
+    if amax is None:
+        amax = (np.abs(rng.normal(0, 1, nb)) * 10.0 ** rng.integers(-6, 6, nb) + 1e-3).astype(np.float32)
     scale = (amax / np.float32(127.0)).astype(np.float32)
     k = rng.integers(-127, 127, (nb, 31)).astype(np.float32)
     v = ((k + np.float32(0.5)) * scale[:, None]).astype(np.float32)
@@ -121,6 +122,28 @@ def test_quantizers_near_ties_bit_exact(dev):
         H.proj_q8(dev, ws, ys, H.ProjInput(x=gx.ptr, xq_out=xo.ptr, xs_out=so.ptr, mode=H.PROJ_F), tokens)
         assert np.array_equal(xo.download(), xq[:tokens])
         assert np.array_equal(so.download().view(np.uint32), xs[:tokens].view(np.uint32))
+
+
+@pytest.mark.parametrize("exponent", [-61, -60, -59, -100, -126, -133, -145])
+def test_quantizers_tiny_scales_bit_exact(dev, exponent):
+    """Near-tie blocks whose scale lies around 2^exponent: below, at and above 2^-60, where halo::CodeScale starts to
+    multiply scale and values by 2^64, and subnormal ones, through both quantizer forms; and blocks whose scale rounds to
+    zero."""
+    rng = np.random.default_rng(-exponent)
+    nb = 3 * 2048 // 32
+    amax = (127.0 * 2.0**exponent * rng.uniform(0.5, 2.0, nb)).astype(np.float32)
+    amax[0] = np.float32(1e-45) * 40  # / 127 rounds to zero
+    x = _near_tie_rows(rng, 3, 2048, amax)
+    xq, xs = O.quantize(x)
+    assert np.abs(xq).max() >= 100 and xs.min() == 0
+    gx = dev.to_device(x)
+    gq, gs = dev.array((3, 2048), np.int8), dev.array((3, 64), np.float32)
+    dev.op("quantize_q8", gx.ptr, gq.ptr, gs.ptr, 3, 2048)
+    assert np.array_equal(gs.download().view(np.uint32), xs.view(np.uint32))
+    assert np.array_equal(gq.download(), xq)
+    ws, ys = [H.Q8Weights(dev, 64, 2048).synth(dev, seed=3)], [dev.array((3, 64), np.float32)]
+    H.proj_q8(dev, ws, ys, H.ProjInput(x=gx.ptr, xq_out=gq.ptr, xs_out=gs.ptr, mode=H.PROJ_F), 3)
+    assert np.array_equal(gq.download(), xq) and np.array_equal(gs.download().view(np.uint32), xs.view(np.uint32))
 
 
 def test_q8x_cols_two_level_bit_exact(dev):
