@@ -191,10 +191,10 @@ int halo_op_attn_prefill(halo_engine* eng, const halo_paged_kv* kv, const halo_p
              -1;
     tiles8 += CeilDiv(g.length, 8);
   }
-  // The tile size that is expected to be done first (16-token tiles need the smaller workspace). Measured at 2 kv heads, in us,
-  // 8-token / 16-token tiles: one prompt of 20 tokens 28 / 33, of 512 65 / 79, 1040 102 / 126, 1800 171 / 186, 2048 208 / 208, 2400
-  // 298 / 239, 8192 2783 / 1703; 256 tokens at position 8192, 1 / 4 / 8 of them, 589 / 694, 690 / 698, 1354 / 840; at position 1000, 200 of 8
-  // tokens 193 / 228, 100 of 12 187 / 126.
+  // The tile size that is expected to be done first (16-token tiles need the smaller workspace). Measured at 2 kv heads,
+  // in us, 8-token / 16-token tiles: one prompt of 20 tokens 28 / 33, of 512 65 / 79, 1040 102 / 126, 1800 171 / 186, 2048
+  // 208 / 208, 2400 298 / 239, 8192 2783 / 1703; 256 tokens at position 8192, 1 / 4 / 8 of them, 589 / 694, 690 / 698,
+  // 1354 / 840; at position 1000, 200 of 8 tokens 193 / 228, 100 of 12 187 / 126.
   std::uint32_t tile = 16;
   std::vector<Tile> tiles = PrefillTiles(segs, nseg, 16);
   const std::uint64_t t16 = BatchTime(tiles, 16, EvenTime(segs, nseg, 16, kv->kv_heads), kv->kv_heads);

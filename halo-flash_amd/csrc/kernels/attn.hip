@@ -727,7 +727,7 @@ extern "C" __global__ void __launch_bounds__(64)
 // One block per CU also means that nothing covers a block's ends: the query row and the first chunk are loaded in one
 // round trip, the gate's values in another, and the last chunk forms no further scores (20 tokens 33 -> 28 us a call, 512
 // tokens 70 -> 65, 400 prompts of 20 tokens 237 -> 168).
-// One 8192-token prompt, 16 heads (550 GFLOP of fp32 products): 3.70 -> 1.73 ms = 318 TFLOP/s (955 of fp16 MFMA issue; a
+// One 8192-token prompt, 16 heads (550 GFLOP of fp32 products): 3.70 -> 1.75 ms = 314 TFLOP/s (943 of fp16 MFMA issue; a
 // large library bf16 matrix product reaches 1380 on this card). The form before held 16 queries per wave, 8 tokens per
 // block, with P through LDS.
 // AttnPrefill<2> (halo_attn_prefill_d2): 8-token tiles, two waves share 32 queries and split the output dims: 0.75x the

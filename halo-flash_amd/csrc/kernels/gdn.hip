@@ -361,7 +361,8 @@ __device__ __forceinline__ void WyPrep(const In* __restrict__ q, const In* __res
 // the products: issued behind them, they take the vector memory pipe as long again as half the products. (Staging the
 // operands in LDS: 515 us for 8000 tokens in slices of 16 columns, 720 us for the ragged batch in slices of 32; this 440
 // and 590.)
-// h varies fastest over the grid: a head's slices land on one XCD (Hv % 8 == 0), whose L2 they share.
+// h varies fastest over the grid: a head's slices land on one XCD (Hv % 8 == 0), whose L2 they share (the time is the same in
+// either order: memory is not what binds).
 template <typename In, int kNC>
 __device__ __forceinline__ void WyScan(const In* __restrict__ k, const float* __restrict__ wy,
                                        const float* __restrict__ Wt, const std::uint32_t* __restrict__ chunks,

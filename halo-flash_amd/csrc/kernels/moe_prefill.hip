@@ -118,7 +118,8 @@ extern "C" __global__ void __launch_bounds__(256)
 }
 
 // grid 1, block 1024: start[e] = exclusive prefix of the group sizes (group e < E: the sum of count[b][e] over the nb
-// partial histograms; group E: T for the shared expert when shared, else 0), and the tile table: groups cut into tiles of `tile` pairs, tiles[i] = {group, first pair, pairs},
+// partial histograms; group E: T for the shared expert when shared, else 0), and the tile table: groups cut
+// into tiles of at most `tile` pairs, tiles[i] = {group, first pair, pairs},
 // ntiles[0] = the tile count. E + 1 <= 1024.
 extern "C" __global__ void __launch_bounds__(1024)
     halo_moe_group_scan(const std::uint32_t* __restrict__ count, std::uint32_t* __restrict__ start,

@@ -911,12 +911,14 @@ __device__ __forceinline__ void GemmTileQ8(const std::int8_t* __restrict__ A0, c
 // 4-byte fp16 scale pairs and fp32 scale pairs), issued by the waves in turn with no register staging; three stage
 // buffers, the loads of stage k + 2 in flight while stage k computes, so one wait and one barrier per stage.
 // Tile rows are 64 bytes with the 16-byte chunk index xor-swizzled by (row >> 2) & 3, which keeps the fragment reads
-// (32 consecutive rows, one chunk each) free of bank conflicts. The stage loop is unrolled by three so every LDS
+// (32 consecutive rows, one chunk each) free of bank conflicts (what conflicts remain, 0.11 of the LDS cycles, are the
+// activation scales', read 8 bytes apart). The stage loop is unrolled by three so every LDS
 // address is a per-lane constant plus an immediate. The scale MFMA is the two-block rank-1 v_mfma_f32_32x32x1_2b,
 // covering two tiles (NMAT * MT even) or both blocks of the stage (a single tile). The activations are the A operand, so
 // that a result register holds one token's values of 32 consecutive matrix rows across its lanes.
-// What bounds it: issue slots. Each 32 x 32 tile and block takes 32 convert / FMA instructions beside its matrix
-// instructions; both together fill 72% of the issue slots at two blocks per CU. (Measured and not kept: products of
+// What bounds it: instruction issue. Each 32 x 32 tile and block takes 32 convert / FMA instructions (128 cycles of a SIMD's
+// vector pipe) beside 64 cycles of the matrix pipe; counted on 8192 x 2048, an instruction of some kind issues in 87% of the
+// SIMDs' cycles at 2048 tokens (vector 69%, matrix pipe busy 30%) and in 97% at 8192 (78%, 35%). (Measured and not kept: products of
 // the next block issued before the current one's additions, 172 VGPRs and one block per CU: 10% slower.) 8192 x 2048 at
 // 8000 tokens: 416 -> 404 us with the activations as A operand (stores of 128 bytes instead of 32).
 // Limits: cols % 64 == 0; every weight offset (rows * qstride) and activation offset fits in 32 bits.
